@@ -58,13 +58,14 @@ void ppm_sweep_kernel(SweepParams P) {
 // kFbTS threads (one thread per interface, the pencil in LDS), with the
 // fallback applied in the reference's cell order; its results replace the
 // sweep kernel's for those pencils.  Launched after every sweep launch; with
-// no flagged group each workgroup only reads the count.
+// no flagged group each workgroup only reads the count (fallback_none).
 template <int UNI, int LEARN, int TS = kFbTS>
 __global__ __launch_bounds__(TS) void ppm_fallback_kernel(SweepParams P) {
   __shared__ double sm[NARR_FB * Cfg<1, TS>::LW];
   PPM_LDS_ENTER(sm);
   DevExec ex;
   const unsigned n = *P.fb_count;
+  if (fallback_none(n)) return;
   for (unsigned k = blockIdx.x; k < n; k += gridDim.x)
     fallback_group<UNI, LEARN, TS>(P, (int)P.fb_list[k], sm, ex);
   fallback_launch_done(P.fb_count, P.fb_done);

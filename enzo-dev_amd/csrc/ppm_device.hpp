@@ -146,6 +146,14 @@ __device__ inline void fallback_group(const SweepParams &P, int grp, double *sm,
   if (threadIdx.x == 0) P.fb_flag[grp] = 0;
 }
 
+// Whether a fallback launch has nothing to do.  Every workgroup of a launch
+// reads the same length (it is cleared only after all of them have counted
+// themselves finished, fallback_launch_done), so with an empty list all of
+// them leave here and none touches the finish count: its atomic adds, one
+// address for up to 512 workgroups, were what an empty launch spent its
+// time on.
+__device__ inline bool fallback_none(unsigned n) { return n == 0u; }
+
 // End of a fallback launch: the last workgroup to finish (every workgroup has
 // read the list length by then) clears the length for the next launch.
 __device__ inline void fallback_launch_done(unsigned *count, unsigned *done) {

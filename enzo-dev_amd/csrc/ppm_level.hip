@@ -137,6 +137,7 @@ __global__ __launch_bounds__(TS) void level_fallback_kernel(const SweepParams *_
   PPM_LDS_ENTER(sm);
   DevExec ex;
   const unsigned n = *count;
+  if (fallback_none(n)) return;
   for (unsigned k = blockIdx.x; k < n; k += gridDim.x) {
     const unsigned e = list[k];
     const int g = grp_grid[e];
