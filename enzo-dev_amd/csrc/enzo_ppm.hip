@@ -34,22 +34,18 @@ using SweepCfg = Cfg<kTP, kTS>;
 
 // ------------------------------------------------------------------------
 // Fused sweep kernel: see ppm_sweep.hpp for the stages.
-template <int UNI, int LEARN>
+template <int UNI, int LEARN, int SV>
 // 5 wavefronts per SIMD: 96 VGPRs (a few spilled) and 31 KB of LDS per
-// workgroup, 5 workgroups per CU
-__global__ __launch_bounds__(kTP *kTS) __attribute__((amdgpu_waves_per_eu(5)))
+// workgroup, 5 workgroups per CU.  The HLL / HLLC tile (SV) keeps more
+// interface values live: 4 wavefronts (116 VGPRs, 6 spilled) take 1.64 ms
+// per 160^3 HLLC step against 1.89 ms with 5 (24 spilled).
+__global__ __launch_bounds__(kTP *kTS) __attribute__((amdgpu_waves_per_eu((SV == 0 ? 5 : 4))))
 void ppm_sweep_kernel(SweepParams P) {
   __shared__ double sm[SweepCfg::SMEM];
   PPM_LDS_ENTER(sm);
   DevExec ex;
   const int tile = xcd_tile((int)blockIdx.x, (int)gridDim.x);
-  TileCounts tc = sweep_tile<kTP, kTS, UNI, DevExec, LEARN>(P, tile, sm, ex);
-  if (threadIdx.x == 0) {
-    // a failing cell or an error: the fallback kernel redoes the group's
-    // pencils whole (the fallback chain can cross segments) and settles them
-    if (tc.bad || tc.err) flag_group(P, tile / P.nseg);
-    if (tc.chains) atomicAdd(&P.counters[1], (unsigned long long)tc.chains);
-  }
+  tile_done<SV>(P, tile, sweep_tile<kTP, kTS, UNI, DevExec, LEARN, SV>(P, tile, sm, ex));
 }
 
 // ------------------------------------------------------------------------
@@ -69,15 +65,6 @@ __global__ __launch_bounds__(TS) void ppm_fallback_kernel(SweepParams P) {
   for (unsigned k = blockIdx.x; k < n; k += gridDim.x)
     fallback_group<UNI, LEARN, TS>(P, (int)P.fb_list[k], sm, ex);
   fallback_launch_done(P.fb_count, P.fb_done);
-}
-
-// ------------------------------------------------------------------------
-// RiemannSolver HLL: every pencil group of the launch on the fallback list
-// (the one-pencil workgroups then take flux_hll's fluxes everywhere).
-__global__ void fb_all_kernel(SweepParams P, unsigned ngroups) {
-  for (unsigned k = blockIdx.x * blockDim.x + threadIdx.x; k < ngroups; k += gridDim.x * blockDim.x)
-    P.fb_list[k] = k;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *P.fb_count = ngroups;
 }
 
 // ------------------------------------------------------------------------
@@ -305,8 +292,8 @@ int check_para(const hipPPMParameter *P) {
   if (P->RiemannSolver != ENZO_PPM_RIEMANN_TWOSHOCK && P->RiemannSolver != ENZO_PPM_RIEMANN_HLL &&
       P->RiemannSolver != ENZO_PPM_RIEMANN_HLLC)
     return ENZO_PPM_ERR_NOT_SUPPORTED;
-  // the HLL and HLLC solvers run in one-pencil workgroups: every swept
-  // pencil must fit
+  // the HLL and HLLC solvers take pencils that a one-pencil workgroup (HLLC's
+  // fallback) holds
   if (P->RiemannSolver != ENZO_PPM_RIEMANN_TWOSHOCK)
     for (int d = 0; d < P->GridRank; d++)
       if (P->GridDimension[d] > kFbTS + 1) {
@@ -541,7 +528,6 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
   S.fb_tag = 0;
   S.tp = kTP;
   S.fb_ok = pencil_fits<kFbTS>(S) ? 1 : 0;
-  S.hll_all = P->RiemannSolver == ENZO_PPM_RIEMANN_HLL ? 1 : 0;
   S.hllc = P->RiemannSolver == ENZO_PPM_RIEMANN_HLLC ? 1 : 0;
   S.learn = D->learned ? D->learn : nullptr;
   if (D->harvest_cap > 0) {
@@ -550,26 +536,23 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
     S.harvest_cap = D->harvest_cap;
     S.harvest_keep = D->harvest_keep;
   }
-  // instantiation by (one cell width, learned start)
+  // instantiation by (one cell width, learned start), or (one cell width)
+  // with the HLL and HLLC solvers, which have no use for the learned start
   const int variant = (S.uni[0] ? 1 : 0) | (D->learned ? 2 : 0);
+  const bool two_shock = P->RiemannSolver == ENZO_PPM_RIEMANN_TWOSHOCK;
   auto launch_main = [&](unsigned nblk) {
     const dim3 g(nblk), b(kTP * kTS);
-    switch (variant) {
-      case 0: hipLaunchKernelGGL((ppm_sweep_kernel<0, 0>), g, b, 0, D->stream, S); break;
-      case 1: hipLaunchKernelGGL((ppm_sweep_kernel<1, 0>), g, b, 0, D->stream, S); break;
-      case 2: hipLaunchKernelGGL((ppm_sweep_kernel<0, 1>), g, b, 0, D->stream, S); break;
-      default: hipLaunchKernelGGL((ppm_sweep_kernel<1, 1>), g, b, 0, D->stream, S); break;
+    if (!two_shock) {
+      if (S.uni[0]) hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 1>), g, b, 0, D->stream, S);
+      else hipLaunchKernelGGL((ppm_sweep_kernel<0, 0, 1>), g, b, 0, D->stream, S);
+      return hipGetLastError();
     }
-    return hipGetLastError();
-  };
-  // the two-shock tiles, or with the HLL solver every group to the
-  // one-pencil workgroups (which then do the whole sweep)
-  const bool whole_pencils = S.hll_all || S.hllc;
-  auto launch_main_or_all = [&](unsigned nblk) {
-    if (!whole_pencils) return launch_main(nblk);
-    const unsigned ngroups = nblk / (unsigned)S.nseg;
-    hipLaunchKernelGGL(fb_all_kernel, dim3((ngroups + 255) / 256), dim3(256), 0, D->stream, S,
-                       ngroups);
+    switch (variant) {
+      case 0: hipLaunchKernelGGL((ppm_sweep_kernel<0, 0, 0>), g, b, 0, D->stream, S); break;
+      case 1: hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 0>), g, b, 0, D->stream, S); break;
+      case 2: hipLaunchKernelGGL((ppm_sweep_kernel<0, 1, 0>), g, b, 0, D->stream, S); break;
+      default: hipLaunchKernelGGL((ppm_sweep_kernel<1, 1, 0>), g, b, 0, D->stream, S); break;
+    }
     return hipGetLastError();
   };
   // one-pencil workgroups: the narrowest width that holds the pencils
@@ -577,8 +560,9 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
   const int fbts = S.fb_ok ? fb_width_of(S) : kFbTS;
   // ngroups: pencil groups of the launch, the most that can be on the list
   // (any number of workgroups is correct: each takes every gridDim-th entry)
-  auto launch_fb = [&](unsigned ngroups) {
-    const unsigned nblk = std::max(1u, std::min(ngroups, fb_blocks(fbts, (whole_pencils ? kFbBlocksWhole : kFbBlocks) * kFbTS)));
+  auto launch_fb = [&](unsigned ngroups) -> hipError_t {
+    if (P->RiemannSolver == ENZO_PPM_RIEMANN_HLL) return hipSuccess;  // no fallback
+    const unsigned nblk = std::max(1u, std::min(ngroups, fb_blocks(fbts, kFbBlocks * kFbTS)));
     return with_fb_width(fbts, [&](auto W) {
       constexpr int TS = decltype(W)::value;
       const dim3 g(nblk), b(TS);
@@ -616,10 +600,9 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
       D->ev_used += 2;
       HIPCHK(hipEventRecord(e0, D->stream));
     }
-    HIPCHK(launch_main_or_all((unsigned)nblk));
-    if (whole_pencils) HIPCHK(launch_fb((unsigned)(nblk / S.nseg)));
+    HIPCHK(launch_main((unsigned)nblk));
     if (D->profile) HIPCHK(hipEventRecord(e1, D->stream));
-    if (!whole_pencils) HIPCHK(launch_fb((unsigned)(nblk / S.nseg)));
+    HIPCHK(launch_fb((unsigned)(nblk / S.nseg)));
   } else {
     // diffusion reads the live transverse velocities of the previous slice
     // (calcdiss.F:207-288 on BaryonField): slices in order, one launch each
@@ -632,7 +615,7 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
     for (int k = 0; k < D->GD[oax]; k++) {
       S.t2_0 = k;
       long long nblk = (long long)S.nseg * S.nblk_t1;
-      HIPCHK(launch_main_or_all((unsigned)nblk));
+      HIPCHK(launch_main((unsigned)nblk));
       HIPCHK(launch_fb((unsigned)S.nblk_t1));  // the next slice reads this one's results
     }
   }

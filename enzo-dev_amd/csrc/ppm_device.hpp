@@ -82,11 +82,8 @@ constexpr int kFbTS = 1024;
 constexpr int kFbWidths[4] = {128, 256, 512, 1024};
 static_assert(kFbWidths[3] == kFbTS, "the widest one-pencil workgroup is kFbTS");
 // The per-cell fallback launches kFbBlocks * kFbTS work-items in all (with
-// no flagged group each workgroup only reads the count); RiemannSolver HLL /
-// HLLC send every group there, kFbBlocksWhole * kFbTS work-items: a CU's
-// worth of LDS per 1024 work-items.
+// no flagged group each workgroup only reads the count).
 constexpr int kFbBlocks = 64;
-constexpr int kFbBlocksWhole = 256;
 
 // narrowest one-pencil width whose tile holds the sweep axis of S (0: none)
 PPM_HD bool pencil_fits_width(const SweepParams &S, int ts) {
@@ -124,6 +121,20 @@ using FbCfg = Cfg<1, kFbTS>;
 __device__ inline void flag_group(const SweepParams &P, int grp) {
   if (atomicExch(&P.fb_flag[grp], 1) == 0)
     P.fb_list[atomicAdd(P.fb_count, 1u)] = P.fb_tag + (unsigned)grp;
+}
+
+// End of a sweep tile: a failing cell or an error puts the tile's pencil
+// group on the fallback list, which redoes the group's pencils whole (the
+// fallback chain can cross segments) and settles them; with the HLL solver
+// there is no fallback and either is an error.
+template <int SV>
+__device__ inline void tile_done(const SweepParams &P, int tile, const TileCounts &tc) {
+  if (threadIdx.x != 0) return;
+  if (tc.bad || tc.err) {
+    if (SV == 0 || P.hllc) flag_group(P, tile / P.nseg);
+    else atomicAdd(&P.counters[2], 1ull);
+  }
+  if (tc.chains) atomicAdd(&P.counters[1], (unsigned long long)tc.chains);
 }
 
 // Every pencil of group `grp` (P.tp pencils along t1) redone whole with the

@@ -58,19 +58,15 @@ constexpr int kShapes = 3;
 constexpr int kShapeTP[kShapes] = {16, 8, 4};
 constexpr int kShapeTS[kShapes] = {16, 32, 64};
 
-template <int TP, int TS, int UNI, int LEARN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5)))
+template <int TP, int TS, int UNI, int LEARN, int SV>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((SV == 0 ? 5 : 4))))
 void level_sweep_kernel(const SweepParams *__restrict__ params, const Work *__restrict__ work) {
   __shared__ double sm[Cfg<TP, TS>::SMEM];
   PPM_LDS_ENTER(sm);
   DevExec ex;
   const Work w = work[xcd_tile((int)blockIdx.x, (int)gridDim.x)];
   const SweepParams &P = params[w.grid];
-  TileCounts tc = sweep_tile<TP, TS, UNI, DevExec, LEARN>(P, w.tile, sm, ex);
-  if (threadIdx.x == 0) {
-    if (tc.bad || tc.err) flag_group(P, w.tile / P.nseg);
-    if (tc.chains) atomicAdd(&P.counters[1], (unsigned long long)tc.chains);
-  }
+  tile_done<SV>(P, w.tile, sweep_tile<TP, TS, UNI, DevExec, LEARN, SV>(P, w.tile, sm, ex));
 }
 
 // The same sweep as one persistent launch: a few workgroups per CU, each
@@ -108,11 +104,7 @@ void level_sweep_persistent_kernel(const SweepParams *__restrict__ params,
     // compiler hoists every tid-derived address of the tile out of the loop
     // and keeps them all live (spilling registers)
     PPM_OPAQUE_VGPR(ex.tid);
-    TileCounts tc = sweep_tile<TP, TS, UNI, DevExec, LEARN>(P, w.tile, sm, ex);
-    if (threadIdx.x == 0) {
-      if (tc.bad || tc.err) flag_group(P, w.tile / P.nseg);
-      if (tc.chains) atomicAdd(&P.counters[1], (unsigned long long)tc.chains);
-    }
+    tile_done<0>(P, w.tile, sweep_tile<TP, TS, UNI, DevExec, LEARN>(P, w.tile, sm, ex));
   }
   if (threadIdx.x == 0) {
     const unsigned nx = gridDim.x / nparts + ((int)(gridDim.x % nparts) > x ? 1u : 0u);
@@ -232,14 +224,6 @@ __global__ void level_periodic_kernel(const BCParams *__restrict__ B) {
     periodic_item(b, gid);
 }
 
-// RiemannSolver HLL / HLLC: the launch's group list onto the fallback list
-__global__ void level_fb_fill_kernel(const unsigned *__restrict__ src, unsigned n, unsigned *list,
-                                     unsigned *count) {
-  for (unsigned k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x)
-    list[k] = src[k];
-  if (blockIdx.x == 0 && threadIdx.x == 0) *count = n;
-}
-
 // one domain face of every grid in the list (blockIdx.y)
 __global__ void level_ext_bc_kernel(const ExtBCParams *__restrict__ B) {
   const ExtBCParams &b = B[blockIdx.y];
@@ -329,11 +313,6 @@ struct hipPPMLevel {
   FlatParams *dflat = nullptr;      // [parity 2][axis 3][grid]
   PresParams *dpres = nullptr;      // [parity 2][grid]
   Work *dwork = nullptr;            // all work lists
-  // RiemannSolver HLL / HLLC: every pencil group goes to the one-pencil
-  // workgroups; per axis and slice, the level-wide group list
-  int whole = 0;
-  unsigned *dfball = nullptr;
-  std::vector<long long> fball_first[3];
   int fb_ts[3] = {kFbTS, kFbTS, kFbTS};  // workgroup width holding every grid's pencils
   Work *dpwork = nullptr;           // pressure chunks
   long long npwork = 0;
@@ -433,7 +412,7 @@ void free_level(hipPPMLevel *L) {
                   L->dtmin, L->counters, L->fb_flag, L->fb_list, L->fb_state, L->grp_grid,
                   L->dgrp_off, L->dparams,
                   L->dflat, L->dpres, L->dwork, L->dpwork, L->learn, L->cws_dt, L->old,
-                  L->dexp, L->dboxes, L->dgeom, L->dfball, L->queues};
+                  L->dexp, L->dboxes, L->dgeom, L->queues};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (L->own_stream && L->stream) (void)hipStreamDestroy(L->stream);
@@ -555,7 +534,6 @@ int build_plan(hipPPMLevel *L) {
   L->hparams.assign((size_t)2 * 3 * G, SweepParams());
   std::vector<FlatParams> hflat((size_t)2 * 3 * G);
   std::vector<Work> work;
-  std::vector<unsigned> fball;
   long long ngroups = 0, nlaunch = 0;
   L->grp_off.assign(G, 0);
   for (int g = 0; g < G; g++) {  // flags per grid: the largest group count of any axis
@@ -645,7 +623,6 @@ int build_plan(hipPPMLevel *L) {
         S.fb_done = L->fb_state + 1;
         S.fb_tag = (unsigned)L->grp_off[g];
         S.fb_ok = pencil_fits<kFbTS>(S) ? 1 : 0;
-        S.hll_all = P0.RiemannSolver == ENZO_PPM_RIEMANN_HLL ? 1 : 0;
         S.hllc = P0.RiemannSolver == ENZO_PPM_RIEMANN_HLLC ? 1 : 0;
         FlatParams &F = hflat[((size_t)par * 3 + d) * G + g];
         memset(&F, 0, sizeof(F));
@@ -674,21 +651,7 @@ int build_plan(hipPPMLevel *L) {
     }
     // work lists: per slice (diffusion) or one, then per (shape, uni)
     const int nslices = L->diffusion ? max_slices : 1;
-    L->fball_first[d].clear();
     for (int k = 0; k < nslices; k++) {
-      L->fball_first[d].push_back((long long)fball.size());
-      if (L->whole)
-        for (int g = 0; g < G; g++) {
-          const SweepParams &S = L->hparams[((size_t)0 * 3 + d) * G + g];
-          if (L->diffusion) {
-            if (k >= S.n_t2) continue;
-            for (int r = 0; r < S.nblk_t1; r++)
-              fball.push_back((unsigned)(L->grp_off[g] + r + (long long)S.nblk_t1 * k));
-          } else {
-            for (long long r = 0; r < (long long)S.nblk_t1 * S.n_t2; r++)
-              fball.push_back((unsigned)(L->grp_off[g] + r));
-          }
-        }
       L->launch_slices[d].push_back((long long)L->launches[d].size());
       for (int s = 0; s < kShapes; s++)
         for (int u = 1; u >= 0; u--) {
@@ -711,7 +674,6 @@ int build_plan(hipPPMLevel *L) {
         }
     }
     L->launch_slices[d].push_back((long long)L->launches[d].size());
-    L->fball_first[d].push_back((long long)fball.size());
   }
   for (int d = 0; d < 3; d++)
     for (int ts : kFbWidths) {  // the narrowest one-pencil width holding every grid's pencils
@@ -747,35 +709,23 @@ int build_plan(hipPPMLevel *L) {
   LCHK(hipMemcpy(L->dflat, hflat.data(), sizeof(FlatParams) * hflat.size(), hipMemcpyHostToDevice));
   if (!work.empty())
     LCHK(hipMemcpy(L->dwork, work.data(), sizeof(Work) * work.size(), hipMemcpyHostToDevice));
-  // whole-pencil group lists: every entry a group of the level, each list no
-  // longer than the fallback list
-  for (int d = 0; d < L->rank; d++)
-    for (size_t k = 0; k + 1 < L->fball_first[d].size(); k++)
-      if (L->fball_first[d][k + 1] - L->fball_first[d][k] > L->ngroups) return ENZO_PPM_ERR_ARGUMENT;
-  for (unsigned e : fball)
-    if ((long long)e >= L->ngroups) return ENZO_PPM_ERR_ARGUMENT;
-  if (L->dfball) (void)hipFree(L->dfball);
-  L->dfball = nullptr;
-  if (dev_alloc(&L->dfball, fball.size())) return ENZO_PPM_ERR_HIP;
   // the persistent launches' counters start at 0 (and their last workgroups
   // leave them at 0)
   if (L->queues) (void)hipFree(L->queues);
   L->queues = nullptr;
   if (dev_alloc(&L->queues, (size_t)std::max(1LL, nlaunch) * 2 * kXCD)) return ENZO_PPM_ERR_HIP;
   LCHK(hipMemset(L->queues, 0, sizeof(unsigned) * (size_t)std::max(1LL, nlaunch) * 2 * kXCD));
-  if (!fball.empty())
-    LCHK(hipMemcpy(L->dfball, fball.data(), sizeof(unsigned) * fball.size(), hipMemcpyHostToDevice));
   drop_graphs(L);
   return ENZO_PPM_SUCCESS;
 }
 
 // the level's fallback launch in one-pencil workgroups of width ts,
-// blocks1024 * kFbTS work-items in all
-// and at most `ngroups` workgroups (the most entries the list can hold)
-hipError_t launch_level_fallback(hipPPMLevel *L, const SweepParams *P, int ts, int blocks1024,
-                                 long long ngroups) {
+// kFbBlocks * kFbTS work-items in all and at most one workgroup per group
+// (the HLL solver has no fallback)
+hipError_t launch_level_fallback(hipPPMLevel *L, const SweepParams *P, int ts) {
+  if (L->para0.RiemannSolver == ENZO_PPM_RIEMANN_HLL) return hipSuccess;
   const unsigned nblk =
-      (unsigned)std::max(1LL, std::min(ngroups, (long long)fb_blocks(ts, blocks1024 * kFbTS)));
+      (unsigned)std::max(1LL, std::min(L->ngroups, (long long)fb_blocks(ts, kFbBlocks * kFbTS)));
   return with_fb_width(ts, [&](auto W) {
     constexpr int TS = decltype(W)::value;
     if (L->learned)
@@ -794,18 +744,9 @@ int launch_level_sweep(hipPPMLevel *L, int d) {
                      0, L->stream,
                      L->dflat + ((size_t)L->parity * 3 + d) * G);
   LCHK(hipGetLastError());
+  const bool two_shock = L->para0.RiemannSolver == ENZO_PPM_RIEMANN_TWOSHOCK;
   const auto &sl = L->launch_slices[d];
   for (size_t k = 0; k + 1 < sl.size(); k++) {
-    if (L->whole) {
-      // HLL / HLLC: every group of the slice to the one-pencil workgroups
-      const long long f0 = L->fball_first[d][k], n = L->fball_first[d][k + 1] - f0;
-      if (n == 0) continue;
-      hipLaunchKernelGGL(level_fb_fill_kernel, dim3((unsigned)std::min<long long>((n + 255) / 256, 1024)),
-                         dim3(256), 0, L->stream, L->dfball + f0, (unsigned)n, L->fb_list, L->fb_state);
-      LCHK(hipGetLastError());
-      LCHK(launch_level_fallback(L, P, L->fb_ts[d], kFbBlocksWhole, n));
-      continue;
-    }
     for (long long li = sl[k]; li < sl[k + 1]; li++) {
       const auto &ln = L->launches[d][li];
       const Work *w = L->dwork + ln.first;
@@ -813,12 +754,15 @@ int launch_level_sweep(hipPPMLevel *L, int d) {
       const dim3 pgrid((unsigned)std::min<long long>(ln.count, L->persistent_blocks));
       unsigned *queue = L->queues + (size_t)2 * kXCD * ln.queue;
       const int nit = (int)ln.count;
+      // HLL and HLLC have no persistent form and no use for the learned start
 #define LEVEL_LAUNCH1(TP, TS, U, LRN)                                                         \
-  if (L->persistent)                                                                        \
+  if (!two_shock)                                                                           \
+    hipLaunchKernelGGL((level_sweep_kernel<TP, TS, U, 0, 1>), grid, blk, 0, L->stream, P, w); \
+  else if (L->persistent)                                                                   \
     hipLaunchKernelGGL((level_sweep_persistent_kernel<TP, TS, U, LRN>), pgrid, blk, 0,       \
                        L->stream, P, w, nit, queue);                                         \
   else                                                                                      \
-    hipLaunchKernelGGL((level_sweep_kernel<TP, TS, U, LRN>), grid, blk, 0, L->stream, P, w);
+    hipLaunchKernelGGL((level_sweep_kernel<TP, TS, U, LRN, 0>), grid, blk, 0, L->stream, P, w);
 #define LEVEL_LAUNCH(S, TP, TS)                                                             \
   if (ln.shape == S) {                                                                    \
     if (L->learned) {                                                                     \
@@ -834,7 +778,7 @@ int launch_level_sweep(hipPPMLevel *L, int d) {
 #undef LEVEL_LAUNCH1
       LCHK(hipGetLastError());
     }
-    LCHK(launch_level_fallback(L, P, L->fb_ts[d], kFbBlocks, L->ngroups));
+    LCHK(launch_level_fallback(L, P, L->fb_ts[d]));
   }
   L->parity ^= 1;
   return ENZO_PPM_SUCCESS;
@@ -894,7 +838,7 @@ int hipPPMLevelCreate(hipPPMLevel **Level, enzo_int NumberOfGrids, const hipPPMP
         P.PPMFlatteningParameter < 0 || P.PPMFlatteningParameter > 3 ||
         (P.PPMDiffusionParameter != 0 && P.PPMDiffusionParameter != 1))
       return ENZO_PPM_ERR_NOT_SUPPORTED;
-    // HLL / HLLC run in one-pencil workgroups: every swept pencil must fit
+    // HLL / HLLC take pencils that a one-pencil workgroup holds
     if (P.RiemannSolver != ENZO_PPM_RIEMANN_TWOSHOCK)
       for (int d = 0; d < P.GridRank; d++)
         if (P.GridDimension[d] > kFbTS + 1) return ENZO_PPM_ERR_NOT_SUPPORTED;
@@ -911,7 +855,6 @@ int hipPPMLevelCreate(hipPPMLevel **Level, enzo_int NumberOfGrids, const hipPPMP
   L->nslot = S_COL0 + L->ncol;
   L->gravity = Para[0].GravityOn != 0;
   L->diffusion = Para[0].PPMDiffusionParameter != 0;
-  L->whole = Para[0].RiemannSolver != ENZO_PPM_RIEMANN_TWOSHOCK ? 1 : 0;
   L->faces.resize(G);
   L->GD.resize(3 * G);
   L->cells.resize(G);

@@ -129,10 +129,9 @@ struct SweepParams {
   unsigned *fb_list, *fb_count, *fb_done;
   unsigned fb_tag;  // added to list entries (the grid's first group in a batched level)
   int fb_ok;        // a one-pencil workgroup holds the whole sweep axis
-  int hll_all;      // RiemannSolver HLL: every cell takes flux_hll's fluxes
-                    // (Grid_xEulerSweep.C:245-256), in one-pencil workgroups
   int hllc;         // RiemannSolver HLLC: flux_hllc's fluxes with its per-cell
-                    // flux_hll fallback (Grid_xEulerSweep.C:258-269), likewise
+                    // flux_hll fallback (Grid_xEulerSweep.C:258-269); without
+                    // it tiles of SV = 1 take flux_hll's fluxes (:245-256)
   int tp;           // pencils per group (the sweep tile's TP)
   // learned two-shock start: network parameters (ppm_learn.hpp), read by
   // the LEARN instantiation only
@@ -190,6 +189,10 @@ constexpr int F_DF = A_DQ, F_EF = A_QL, F_UF = A_QR, F_VF = A_Q6, F_WF = A_ST,
 // work-item reads its own interface's entries before it stores that
 // interface's fluxes into F_UB = A_X); C_l is computed again
 constexpr int A_AC_R = A_COL, A_AC_P = A_X;
+// the second gas-energy source term of the HLL and HLLC tiles (the first is
+// in F_UB): the sound speeds are spent once the characteristics are in
+// registers
+constexpr int F_GB = A_CS;
 
 // Fallback workgroups (one pencil, TP = 1) keep two more arrays: the HLL
 // density flux for the in-order fallback decision, then the two gas-energy
@@ -268,8 +271,9 @@ struct Regs {
   // two-shock fluxes
   double h_df, h_uf, h_vf, h_wf, h_ef, h_gef, h_sl, h_sr, h_bm0, h_bp0;
   int hll;
-  // HLLC workgroups: the HLLC weights of the interface, the gas-energy
-  // source terms sl*gesl and sr*gesr, and the cell's gas-energy source
+  // HLL / HLLC tiles and HLLC fallback workgroups: the solver's weights of
+  // the interface, the gas-energy source terms sl*gesl and sr*gesr, and (in
+  // the workgroups) the cell's gas-energy source
   double c_sl, c_sr, c_ga, c_gb, c_ges;
 };
 
@@ -1020,6 +1024,26 @@ PPM_HD void hllc_flux(const HllIn &h, Regs &r) {
   }
   r.c_sl = sl;
   r.c_sr = sr;
+  r.h_bm0 = bm0;
+  r.h_bp0 = bp0;
+}
+
+// the diffusion terms of an interface's HLL / HLLC fluxes (flux_hll.F:166-195)
+// from its diffusion coefficient dc
+template <int TP, int TS, int UNI = 0>
+PPM_HD void hll_diffusion(const SweepParams &P, const Tile &T, double *sm, int p, int i, double dc,
+                          HllIn &h) {
+  h.diffd = h.diffuu = h.diffuv = h.diffuw = h.diffue = h.diffuge = 0.0;
+  if (P.idiff == 0) return;
+  const int ca = i - 1 - T.L0, cb = i - T.L0;
+  const double da = LDS<TP, TS, UNI>(sm, A_D, p, ca), dbb = LDS<TP, TS, UNI>(sm, A_D, p, cb);
+  h.diffd = dc * (da - dbb);
+  h.diffuu = dc * (da * LDS<TP, TS, UNI>(sm, A_U, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_U, p, cb));
+  h.diffuv = dc * (da * LDS<TP, TS, UNI>(sm, A_V, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_V, p, cb));
+  h.diffuw = dc * (da * LDS<TP, TS, UNI>(sm, A_W, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_W, p, cb));
+  h.diffue = dc * (da * LDS<TP, TS, UNI>(sm, A_E, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_E, p, cb));
+  if (P.idual == 1)
+    h.diffuge = dc * (da * LDS<TP, TS, UNI>(sm, A_GE, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_GE, p, cb));
 }
 
 // Phase: Eulerian corrections (inteuler.F:321-551), two-shock solve and
@@ -1029,7 +1053,8 @@ PPM_HD void hllc_flux(const HllIn &h, Regs &r) {
 // network's evaluation: STAGE 0 computes the two-shock inputs into Regs,
 // STAGE 1 continues from them (with Regs::ls / lc, the interface's network
 // correction).
-template <int TP, int TS, int UNI = 0, int FB = 0, int LEARN = 0, int STAGE = 2>
+// SV 0: the two-shock solver; 1: HLL or HLLC (P.hllc) fluxes in its place.
+template <int TP, int TS, int UNI = 0, int FB = 0, int LEARN = 0, int STAGE = 2, int SV = 0>
 PPM_HD void ph_solve(const SweepParams &P, const Tile &T, double *sm, int tid, Regs &r) {
   int p = tid / TS, q = tid % TS;
   if constexpr (FB != 0 && STAGE != 1) r.hll = 0;
@@ -1137,6 +1162,30 @@ PPM_HD void ph_solve(const SweepParams &P, const Tile &T, double *sm, int tid, R
     uls = r.s_ul;
     urs = r.s_ur;
   }
+  if constexpr (SV != 0) {
+    // flux_hll.F / flux_hllc.F on the interface states (both pressures pmin
+    // when pressure-free, as the two-shock solver leaves them)
+    if (P.ipresfree == 1) pls = prs = P.pmin;
+    HllIn h;
+    h.dls = dls; h.drs = drs; h.pls = pls; h.prs = prs; h.uls = uls; h.urs = urs;
+    h.vls = r.vls; h.vrs = r.vrs; h.wls = r.wls; h.wrs = r.wrs; h.gels = r.gels; h.gers = r.gers;
+    hll_diffusion<TP, TS, UNI>(
+        P, T, sm, p, i, P.idiff != 0 ? diffcoef1<TP, TS, UNI>(P, T, sm, p, i) : 0.0, h);
+    h.gamma = gamma;
+    h.qc = qc_of<UNI>(P, T, i);
+    h.idual = P.idual;
+    if (P.hllc) {
+      hllc_flux(h, r);
+    } else {
+      hll_flux(h, r);
+      r.df = r.h_df; r.ef = r.h_ef; r.uf = r.h_uf; r.vf = r.h_vf; r.wf = r.h_wf; r.gef = r.h_gef;
+      r.c_sl = r.h_sl;
+      r.c_sr = r.h_sr;
+      r.c_ga = r.h_sl * r.h_bm0;
+      r.c_gb = r.h_sr * r.h_bp0;
+    }
+    return;
+  }
   // two-shock solution
   double pbar, ubar, ps0;
   const double pls_in = pls, prs_in = prs;
@@ -1222,17 +1271,7 @@ PPM_HD void ph_solve(const SweepParams &P, const Tile &T, double *sm, int tid, R
     HllIn h;
     h.dls = dls; h.drs = drs; h.pls = pls; h.prs = prs; h.uls = uls; h.urs = urs;
     h.vls = r.vls; h.vrs = r.vrs; h.wls = r.wls; h.wrs = r.wrs; h.gels = r.gels; h.gers = r.gers;
-    h.diffd = h.diffuu = h.diffuv = h.diffuw = h.diffue = h.diffuge = 0.0;
-    if (P.idiff != 0) {  // flux_hll.F:166-195
-      const double da = LDS<TP, TS, UNI>(sm, A_D, p, ca), dbb = LDS<TP, TS, UNI>(sm, A_D, p, cb);
-      h.diffd = dc * (da - dbb);
-      h.diffuu = dc * (da * LDS<TP, TS, UNI>(sm, A_U, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_U, p, cb));
-      h.diffuv = dc * (da * LDS<TP, TS, UNI>(sm, A_V, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_V, p, cb));
-      h.diffuw = dc * (da * LDS<TP, TS, UNI>(sm, A_W, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_W, p, cb));
-      h.diffue = dc * (da * LDS<TP, TS, UNI>(sm, A_E, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_E, p, cb));
-      if (P.idual == 1)
-        h.diffuge = dc * (da * LDS<TP, TS, UNI>(sm, A_GE, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_GE, p, cb));
-    }
+    hll_diffusion<TP, TS, UNI>(P, T, sm, p, i, dc, h);
     h.gamma = gamma;
     h.qc = qc;
     h.idual = P.idual;
@@ -1242,7 +1281,7 @@ PPM_HD void ph_solve(const SweepParams &P, const Tile &T, double *sm, int tid, R
 }
 
 // Phase: store the interface fluxes into LDS (indexed by the right cell).
-template <int TP, int TS, int UNI = 0, int FB = 0>
+template <int TP, int TS, int UNI = 0, int FB = 0, int SV = 0>
 PPM_HD void ph_store_flux(const SweepParams &P, const Tile &T, double *sm, int tid,
                           const Regs &r) {
   (void)P;
@@ -1256,7 +1295,12 @@ PPM_HD void ph_store_flux(const SweepParams &P, const Tile &T, double *sm, int t
   LDS<TP, TS, UNI>(sm, F_VF, p, cb) = r.vf;
   LDS<TP, TS, UNI>(sm, F_WF, p, cb) = r.wf;
   LDS<TP, TS, UNI>(sm, F_GEF, p, cb) = r.gef;
-  LDS<TP, TS, UNI>(sm, F_UB, p, cb) = r.ub;
+  if constexpr (SV != 0) {
+    LDS<TP, TS, UNI>(sm, F_UB, p, cb) = r.c_ga;
+    LDS<TP, TS, UNI>(sm, F_GB, p, cb) = r.c_gb;
+  } else {
+    LDS<TP, TS, UNI>(sm, F_UB, p, cb) = r.ub;
+  }
   if constexpr (FB != 0) {
     if (P.hllc) {  // the HLLC gas-energy source terms (F_UB is unused here)
       LDS<TP, TS, UNI>(sm, F_UB, p, cb) = r.c_ga;
@@ -1300,9 +1344,10 @@ PPM_HD void upd_range(const SweepParams &P, const Tile &T, int &c0, int &c1) {
   c1 = T.IB - 1 < P.i2 ? T.IB - 1 : P.i2;
 }
 
-// Phase: negative density / energy check (flux_twoshock.F:401-403).
-// Returns the number of failing cells seen by this thread.
-template <int TP, int TS, int UNI = 0>
+// Phase: negative density / energy check (flux_twoshock.F:401-403; the HLL
+// and HLLC solvers check the density alone, flux_hll.F:349-351 and
+// flux_hllc.F:344).  Returns the number of failing cells seen by this thread.
+template <int TP, int TS, int UNI = 0, int SV = 0>
 PPM_HD int ph_check(const SweepParams &P, const Tile &T, double *sm, int tid) {
   int c0, c1;
   upd_range(P, T, c0, c1);
@@ -1314,7 +1359,7 @@ PPM_HD int ph_check(const SweepParams &P, const Tile &T, double *sm, int tid) {
     int c = cell - T.L0;
     double d = LDS<TP, TS, UNI>(sm, A_D, p, c), e = LDS<TP, TS, UNI>(sm, A_E, p, c);
     double dfl = LDS<TP, TS, UNI>(sm, F_DF, p, c), dfr = LDS<TP, TS, UNI>(sm, F_DF, p, c + 1);
-    if (d + (dfl - dfr) <= 0.0 || e < 0.0) bad++;
+    if (SV != 0 ? (d + dfl) - dfr <= 0.0 : (d + (dfl - dfr) <= 0.0 || e < 0.0)) bad++;
   }
   return bad;
 }
@@ -1339,19 +1384,6 @@ PPM_HD int ph_fb_decide(const SweepParams &P, const Tile &T, double *sm, int tid
   int nfb = 0, err = 0, prev = 0;
   LDS<TP, TS, UNI>(sm, A_COL, 0, P.i1 - 1 - T.L0) = 0.0;
   LDS<TP, TS, UNI>(sm, A_COL, 0, P.i2 + 1 - T.L0) = 0.0;
-  if (P.hll_all) {
-    // the HLL solver on the whole pencil: every interface takes the HLL
-    // fluxes and flux_hll's own check (flux_hll.F:336-384) is the only one;
-    // no cell counts as a fallback
-    for (int cell = P.i1; cell <= P.i2; cell++) {
-      const int c = cell - T.L0;
-      LDS<TP, TS, UNI>(sm, A_COL, 0, c) = 1.0;
-      if ((LDS<TP, TS, UNI>(sm, A_D, 0, c) + LDSH<TP, TS, UNI>(sm, A_HA, c)) -
-              LDSH<TP, TS, UNI>(sm, A_HA, c + 1) <= 0.0)
-        err = 1;
-    }
-    return err ? kFbError : 0;
-  }
   for (int cell = P.i1; cell <= P.i2; cell++) {
     const int c = cell - T.L0;
     const double d = LDS<TP, TS, UNI>(sm, A_D, 0, c), e = LDS<TP, TS, UNI>(sm, A_E, 0, c);
@@ -1406,7 +1438,7 @@ PPM_HD void ph_fb_apply(const SweepParams &P, const Tile &T, double *sm, int tid
 // For a cell c+1 after a fallback at c alone, the reference's one-cell call
 // evaluates that at c+2 from locals it never set (flux_hll.F:304-307 with
 // i2 = c); here they are the HLL terms of interface c+2, as in the oracle.
-template <int TP, int TS, int UNI = 0, int FB = 0>
+template <int TP, int TS, int UNI = 0, int FB = 0, int SV = 0>
 PPM_HD int ph_euler(const SweepParams &P, const Tile &T, double *sm, int tid, bool fbon = false) {
   int c0, c1;
   upd_range(P, T, c0, c1);
@@ -1436,7 +1468,13 @@ PPM_HD int ph_euler(const SweepParams &P, const Tile &T, double *sm, int tid, bo
       double ge = LDS<TP, TS, UNI>(sm, A_GE, p, c);
       double pcent = fmx((gamma - 1.0) * ge * d, kTiny);
       double qc = qc_of<UNI>(P, T, cell);
-      double ges = qc * pcent * (LDS<TP, TS, UNI>(sm, F_UB, p, c) - LDS<TP, TS, UNI>(sm, F_UB, p, c + 1));
+      double ges;
+      if constexpr (SV != 0)  // flux_hll.F:297-308, flux_hllc.F:306-316
+        ges = qc * pcent *
+              (LDS<TP, TS, UNI>(sm, F_UB, p, c) + LDS<TP, TS, UNI>(sm, F_GB, p, c) -
+               LDS<TP, TS, UNI>(sm, F_UB, p, c + 1) - LDS<TP, TS, UNI>(sm, F_GB, p, c + 1));
+      else
+        ges = qc * pcent * (LDS<TP, TS, UNI>(sm, F_UB, p, c) - LDS<TP, TS, UNI>(sm, F_UB, p, c + 1));
       if constexpr (FB != 0) {
         if (P.hllc) ges = LDS<TP, TS, UNI>(sm, F_UB, p, c);  // ph_hllc_ges
         if (fbon &&
@@ -1600,7 +1638,7 @@ PPM_HD void ph_load_col(const SweepParams &P, const Tile &T, double *sm, int tid
 // Phase: colour interface state and flux (inteuler.F:437-450, 493-551;
 // flux_twoshock.F:251-259, 375-380; euler.F:173-177 division by dx),
 // stored as colf/dx into F_COLF, and captured for owned faces.
-template <int TP, int TS, int UNI = 0, int FB = 0>
+template <int TP, int TS, int UNI = 0, int FB = 0, int SV = 0>
 PPM_HD void ph_col_flux(const SweepParams &P, const Tile &T, double *sm, int tid, int n,
                         const Regs &r) {
   int p = tid / TS, q = tid % TS;
@@ -1616,13 +1654,18 @@ PPM_HD void ph_col_flux(const SweepParams &P, const Tile &T, double *sm, int tid
   if (r.ovr) colrs = colrs * r.dra / r.drs_pre;
   colls = fmx(colls, kColorFloor);
   colrs = fmx(colrs, kColorFloor);
-  const bool up = r.ub > 0.0;
-  double colb = (up ? colls : colrs) * r.db / (up ? r.dls : r.drs);
-  double colf = T.dt * r.ub * colb;
-  if (FB != 0 && r.hll)  // flux_hll.F:231-236, 272-276, 327-331
-    colf = T.dt * (r.h_sl * (r.h_bm0 * colls) + r.h_sr * (r.h_bp0 * colrs));
-  else if (FB != 0 && P.hllc)  // flux_hllc.F:252-258, 286-290, 336-340
+  double colf;
+  if constexpr (SV != 0) {  // flux_hll.F:231-236, 272-276, 327-331 and flux_hllc.F likewise
     colf = T.dt * (r.c_sl * (r.h_bm0 * colls) + r.c_sr * (r.h_bp0 * colrs));
+  } else {
+    const bool up = r.ub > 0.0;
+    double colb = (up ? colls : colrs) * r.db / (up ? r.dls : r.drs);
+    colf = T.dt * r.ub * colb;
+    if (FB != 0 && r.hll)  // flux_hll.F:231-236, 272-276, 327-331
+      colf = T.dt * (r.h_sl * (r.h_bm0 * colls) + r.h_sr * (r.h_bp0 * colrs));
+    else if (FB != 0 && P.hllc)  // flux_hllc.F:252-258, 286-290, 336-340
+      colf = T.dt * (r.c_sl * (r.h_bm0 * colls) + r.c_sr * (r.h_bp0 * colrs));
+  }
   colf = (UNI && P.dx_pow2) ? colf * P.inv_dx : colf / TS_<UNI>(P, T_DX, i);
   LDS<TP, TS, UNI>(sm, F_COLF, p, cb) = colf;
   if (P.face_head && i >= T.o && i < T.o + T.w) {
@@ -1880,7 +1923,7 @@ PPM_HD void sweep_var(const SweepParams &P, const Tile &T, double *sm, X &ex) {
   ex.run([&](int tid, Regs &r) { ph_iface<V, TP, TS, UNI>(P, T, sm, tid, r); });
 }
 
-template <int TP, int TS, int UNI, int FB, class X, int LEARN = 0>
+template <int TP, int TS, int UNI, int FB, class X, int LEARN = 0, int SV = 0>
 PPM_HD TileCounts sweep_body(const SweepParams &P, const Tile &T, double *sm, X &ex) {
   TileCounts tc;
   tc.nfb = 0;
@@ -1912,8 +1955,8 @@ PPM_HD TileCounts sweep_body(const SweepParams &P, const Tile &T, double *sm, X 
     });
   } else {
     ex.run([&](int tid, Regs &r) {
-      ph_solve<TP, TS, UNI, FB, LEARN>(P, T, sm, tid, r);
-      ph_store_flux<TP, TS, UNI, FB>(P, T, sm, tid, r);
+      ph_solve<TP, TS, UNI, FB, LEARN, 2, SV>(P, T, sm, tid, r);
+      ph_store_flux<TP, TS, UNI, FB, SV>(P, T, sm, tid, r);
     });
   }
   if constexpr (FB != 0) {
@@ -1922,25 +1965,25 @@ PPM_HD TileCounts sweep_body(const SweepParams &P, const Tile &T, double *sm, X 
       ex.run([&](int tid, Regs &r) { ph_hllc_ges_store<TP, TS, UNI>(P, T, sm, tid, r); });
     }
   }
-  tc.bad = ex.count([&](int tid, Regs &r) { (void)r; return ph_check<TP, TS, UNI>(P, T, sm, tid); });
+  tc.bad = ex.count([&](int tid, Regs &r) { (void)r; return ph_check<TP, TS, UNI, SV>(P, T, sm, tid); });
   bool fbon = false;
   int fberr = 0;
   if constexpr (FB != 0) {
-    if (tc.bad || P.hll_all || P.hllc) {  // block-uniform
+    if (tc.bad || P.hllc) {  // block-uniform
     const int dec = ex.first([&](int tid, Regs &r) {
       (void)r;
       return ph_fb_decide<TP, TS, UNI>(P, T, sm, tid);
     });
     tc.nfb = dec % kFbError;
     fberr = dec / kFbError;
-    fbon = tc.nfb > 0 || P.hll_all;
+    fbon = tc.nfb > 0;
     if (fbon) ex.run([&](int tid, Regs &r) { ph_fb_apply<TP, TS, UNI>(P, T, sm, tid, r); });
     }
   }
   tc.err = ex.count([&](int tid, Regs &r) {
     (void)r;
     ph_capture<TP, TS, UNI>(P, T, sm, tid);
-    return ph_euler<TP, TS, UNI, FB>(P, T, sm, tid, fbon);
+    return ph_euler<TP, TS, UNI, FB, SV>(P, T, sm, tid, fbon);
   });
   tc.err += fberr;
   if (P.idual) ex.run([&](int tid, Regs &r) { (void)r; ph_pgas_spec<TP, TS, UNI>(P, T, sm, tid); });
@@ -1950,7 +1993,7 @@ PPM_HD TileCounts sweep_body(const SweepParams &P, const Tile &T, double *sm, X 
     ex.run([&](int tid, Regs &r) { (void)r; ph_load_col<TP, TS, UNI>(P, T, sm, tid, n); });
     ex.run([&](int tid, Regs &r) { (void)r; ph_slope<TP, TS, UNI>(P, T, sm, tid, A_COL); });
     ex.run([&](int tid, Regs &r) { ph_parab<TP, TS, UNI>(P, T, sm, tid, A_COL, 0, r); });
-    ex.run([&](int tid, Regs &r) { ph_col_flux<TP, TS, UNI, FB>(P, T, sm, tid, n, r); });
+    ex.run([&](int tid, Regs &r) { ph_col_flux<TP, TS, UNI, FB, SV>(P, T, sm, tid, n, r); });
     ex.run([&](int tid, Regs &r) { (void)r; ph_col_update<TP, TS, UNI>(P, T, sm, tid, n); });
   }
   return tc;
@@ -1958,10 +2001,18 @@ PPM_HD TileCounts sweep_body(const SweepParams &P, const Tile &T, double *sm, X 
 
 // A tile of the main launch.  bad > 0 means some cell of the tile needs the
 // fallback (or, without it, is an error); its pencils are then redone by a
-// fallback workgroup, which also settles the errors of those pencils.
-template <int TP, int TS, int UNI, class X, int LEARN = 0>
+// fallback workgroup, which also settles the errors of those pencils.  With
+// the HLL solver (SV 1, P.hllc 0) there is no fallback: bad is an error.
+//
+// HLL and HLLC (SV 1) run in the same tiles as the two-shock solver: every
+// cell's update needs its own interfaces' fluxes only, and the phases around
+// the solver are shared.  At 144x96x131 the HLL sweep takes 178 us (one
+// workgroup per pencil, which held it whole and solved the two-shock problem
+// first: 1,310 us), at 160^3 with two colours the HLLC sweep 510 us
+// (3,980 us).
+template <int TP, int TS, int UNI, class X, int LEARN = 0, int SV = 0>
 PPM_HD TileCounts sweep_tile(const SweepParams &P, int block, double *sm, X &ex) {
-  return sweep_body<TP, TS, UNI, 0, X, LEARN>(P, make_tile<TP, TS, UNI>(P, block), sm, ex);
+  return sweep_body<TP, TS, UNI, 0, X, LEARN, SV>(P, make_tile<TP, TS, UNI>(P, block), sm, ex);
 }
 
 // One whole pencil in a one-pencil workgroup of TS threads, with the

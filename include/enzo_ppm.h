@@ -158,11 +158,9 @@ typedef struct hipPPMData hipPPMData;
    fallback when RiemannSolverFallback is set, HLL (1): flux_hll over whole
    pencils (Grid_xEulerSweep.C:245-256), its negative-density check giving
    ENZO_PPM_ERR_NEGATIVE, or HLLC (4): flux_hllc (:258-269) with its own
-   per-cell flux_hll fallback; with HLL or HLLC each pencil is computed by
-   one workgroup that holds it whole, so pencils of up to 1025 cells.  The
-   others: ENZO_PPM_ERR_NOT_SUPPORTED.  The batched level
-   (hipPPMLevelCreate) takes the same three; with HLL or HLLC every pencil
-   group of the level goes to the one-pencil workgroups. */
+   per-cell flux_hll fallback; HLL and HLLC take pencils of up to 1025
+   cells.  The others: ENZO_PPM_ERR_NOT_SUPPORTED.  The batched level
+   (hipPPMLevelCreate) takes the same three. */
 int hipPPMInitParameter(hipPPMParameter *Para, enzo_int DensNum, enzo_int TENum,
                         enzo_int Vel1Num, enzo_int Vel2Num, enzo_int Vel3Num,
                         enzo_int GENum, enzo_int MaxNumberOfBaryonFields,
