@@ -34,7 +34,10 @@ using SweepCfg = Cfg<kTP, kTS>;
 
 // ------------------------------------------------------------------------
 // Fused sweep kernel: see ppm_sweep.hpp for the stages.
-template <int UNI, int LEARN, int SV>
+// DF 1: diffusion in one launch (wait_pair).  DF 0 keeps the tile's test of
+// P.idiff, never set there: it splits the Riemann phase, which the compiler
+// then schedules better (256^3 step 7.50 ms; 7.70 without the test).
+template <int UNI, int LEARN, int SV, int DF>
 // 5 wavefronts per SIMD: 96 VGPRs (a few spilled) and 31 KB of LDS per
 // workgroup, 5 workgroups per CU.  The HLL / HLLC tile (SV) keeps more
 // interface values live: 4 wavefronts (116 VGPRs, 6 spilled) take 1.64 ms
@@ -44,8 +47,16 @@ void ppm_sweep_kernel(SweepParams P) {
   __shared__ double sm[SweepCfg::SMEM];
   PPM_LDS_ENTER(sm);
   DevExec ex;
-  const int tile = xcd_tile((int)blockIdx.x, (int)gridDim.x);
-  tile_done<SV>(P, tile, sweep_tile<kTP, kTS, UNI, DevExec, LEARN, SV>(P, tile, sm, ex));
+  int tile;
+  if constexpr (DF == 0) {
+    tile = xcd_tile((int)blockIdx.x, (int)gridDim.x);
+  } else {  // slices in order (wait_pair)
+    __shared__ int turn;
+    if (threadIdx.x == 0) turn = (int)atomicAdd(P.ticket, 1u);
+    __syncthreads();
+    tile = PPM_UNIFORM(turn);
+  }
+  tile_done<SV>(P, tile, sweep_tile<kTP, kTS, UNI, DevExec, LEARN, SV, DF == 0 ? -1 : DF>(P, tile, sm, ex));
 }
 
 // ------------------------------------------------------------------------
@@ -70,7 +81,11 @@ __global__ __launch_bounds__(TS) void ppm_fallback_kernel(SweepParams P) {
 // ------------------------------------------------------------------------
 // Per-sweep preparation (prep_item in ppm_device.hpp), one item per thread.
 __global__ void sweep_prep_kernel(FlatParams F) {
-  prep_item(F, (long long)blockIdx.x * blockDim.x + threadIdx.x);
+  const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  prep_item(F, gid);
+  if (F.unpublished)  // diffusion in one launch
+    for (long long g = gid; g < F.cells; g += (long long)gridDim.x * blockDim.x)
+      F.unpublished[g] = __longlong_as_double((long long)kUnpublished);
 }
 
 // ------------------------------------------------------------------------
@@ -195,6 +210,7 @@ struct hipPPMData {
   bool gravity = false;
   double *A = nullptr, *B = nullptr;
   double *pres = nullptr;
+  double *xch = nullptr;    // diffusion: the slices' exchange (wait_pair), if there is memory for it
   double *accel = nullptr;  // 3 * cells when gravity
   const double *accel_ext[3] = {nullptr, nullptr, nullptr};  // the caller's (no-alloc entry)
   double *tab[3] = {nullptr, nullptr, nullptr};
@@ -207,7 +223,7 @@ struct hipPPMData {
   unsigned long long *counters = nullptr;  // [0] fallback [1] DE chain [2] errors [3] unsupported
   // per-cell fallback: group flags, flagged-group list, {count, done}
   int *fb_flag = nullptr;
-  unsigned *fb_list = nullptr, *fb_state = nullptr;
+  unsigned *fb_list = nullptr, *fb_state = nullptr;  // fb_state: count, done, diffusion's ticket
   long long fb_groups = 0;
   int *segbuf = nullptr;  // per axis: o[nseg], w[nseg]
   int uni[3] = {0, 0, 0};  // axis has one cell width
@@ -324,7 +340,7 @@ void free_data(hipPPMData *D) {
   if (!D) return;
   for (hipEvent_t e : D->ev) (void)hipEventDestroy(e);
   D->ev.clear();
-  void *ptrs[] = {D->A, D->B, D->pres, D->accel, D->tab[0], D->tab[1], D->tab[2], D->cwdev[0],
+  void *ptrs[] = {D->A, D->B, D->pres, D->xch, D->accel, D->tab[0], D->tab[1], D->tab[2], D->cwdev[0],
                   D->cwdev[1], D->cwdev[2], D->flat, D->qc, D->dt, D->dtmin, D->counters, D->segbuf,
                   D->fb_flag, D->fb_list, D->fb_state, D->learn, D->harvest, D->harvest_n,
                   D->cwdt[0], D->cwdt[1], D->cwdt[2], D->old,
@@ -469,7 +485,12 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
     F.dt = dtFixed;
     F.dtp = dtp;
     F.qc = D->qc;
+    const bool pipe = P->PPMDiffusionParameter != 0;
+    F.unpublished = !pipe || oax >= rank ? nullptr
+                    : D->xch ? D->xch : D->B + (long long)(S_VX + oax) * D->cells;
+    F.ticket = pipe ? D->fb_state + 2 : nullptr;
     long long n = N + (iflat ? (long long)(i2 - i1 + 3) * F.n_outer : 0);
+    if (F.unpublished) n = std::max(n, std::min(D->cells, 256LL * 2048));
     hipLaunchKernelGGL(sweep_prep_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                        D->stream, F);
     HIPCHK(hipGetLastError());
@@ -540,18 +561,19 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
   // with the HLL and HLLC solvers, which have no use for the learned start
   const int variant = (S.uni[0] ? 1 : 0) | (D->learned ? 2 : 0);
   const bool two_shock = P->RiemannSolver == ENZO_PPM_RIEMANN_TWOSHOCK;
-  auto launch_main = [&](unsigned nblk) {
+  auto launch_tiles = [&](unsigned nblk, auto diff) {
+    constexpr int DF = decltype(diff)::value;
     const dim3 g(nblk), b(kTP * kTS);
     if (!two_shock) {
-      if (S.uni[0]) hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 1>), g, b, 0, D->stream, S);
-      else hipLaunchKernelGGL((ppm_sweep_kernel<0, 0, 1>), g, b, 0, D->stream, S);
+      if (S.uni[0]) hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 1, DF>), g, b, 0, D->stream, S);
+      else hipLaunchKernelGGL((ppm_sweep_kernel<0, 0, 1, DF>), g, b, 0, D->stream, S);
       return hipGetLastError();
     }
     switch (variant) {
-      case 0: hipLaunchKernelGGL((ppm_sweep_kernel<0, 0, 0>), g, b, 0, D->stream, S); break;
-      case 1: hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 0>), g, b, 0, D->stream, S); break;
-      case 2: hipLaunchKernelGGL((ppm_sweep_kernel<0, 1, 0>), g, b, 0, D->stream, S); break;
-      default: hipLaunchKernelGGL((ppm_sweep_kernel<1, 1, 0>), g, b, 0, D->stream, S); break;
+      case 0: hipLaunchKernelGGL((ppm_sweep_kernel<0, 0, 0, DF>), g, b, 0, D->stream, S); break;
+      case 1: hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 0, DF>), g, b, 0, D->stream, S); break;
+      case 2: hipLaunchKernelGGL((ppm_sweep_kernel<0, 1, 0, DF>), g, b, 0, D->stream, S); break;
+      default: hipLaunchKernelGGL((ppm_sweep_kernel<1, 1, 0, DF>), g, b, 0, D->stream, S); break;
     }
     return hipGetLastError();
   };
@@ -574,51 +596,50 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
       }
     });
   };
-  if (S.idiff == 0) {
-    // all pencils at once: t1 is the contiguous transverse axis for y/z
-    // sweeps (coalesced loads), the row axis for x sweeps
-    if (dim == 0) { S.ax_t1 = 1; S.ax_t2 = 2; }
-    else if (dim == 1) { S.ax_t1 = 0; S.ax_t2 = 2; }
-    else { S.ax_t1 = 0; S.ax_t2 = 1; }
-    S.n_t1 = D->GD[S.ax_t1];
-    S.n_t2 = D->GD[S.ax_t2];
-    S.t2_0 = 0;
-    set_strides(S);
-    S.nblk_t1 = (S.n_t1 + kTP - 1) / kTP;
-    long long nblk = (long long)S.nseg * S.nblk_t1 * S.n_t2;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (D->profile) {
-      if (D->ev_used + 2 > D->ev.size()) {
-        for (int k = 0; k < 2; k++) {
-          hipEvent_t e;
-          HIPCHK(hipEventCreate(&e));
-          D->ev.push_back(e);
-        }
-      }
-      e0 = D->ev[D->ev_used];
-      e1 = D->ev[D->ev_used + 1];
-      D->ev_used += 2;
-      HIPCHK(hipEventRecord(e0, D->stream));
-    }
-    HIPCHK(launch_main((unsigned)nblk));
-    if (D->profile) HIPCHK(hipEventRecord(e1, D->stream));
-    HIPCHK(launch_fb((unsigned)(nblk / S.nseg)));
-  } else {
-    // diffusion reads the live transverse velocities of the previous slice
-    // (calcdiss.F:207-288 on BaryonField): slices in order, one launch each
+  // all pencils at once.  Without diffusion t1 is the contiguous transverse
+  // axis for y/z sweeps (coalesced loads), the row axis for x sweeps; with it
+  // t2 is the slice axis, whose slices wait for each other (wait_pair)
+  S.pipe = S.idiff != 0;
+  if (S.pipe) {
     S.ax_t1 = rax;
     S.ax_t2 = oax;
-    S.n_t1 = D->GD[rax];
-    S.n_t2 = 1;
-    set_strides(S);
-    S.nblk_t1 = (S.n_t1 + kTP - 1) / kTP;
-    for (int k = 0; k < D->GD[oax]; k++) {
-      S.t2_0 = k;
-      long long nblk = (long long)S.nseg * S.nblk_t1;
-      HIPCHK(launch_main((unsigned)nblk));
-      HIPCHK(launch_fb((unsigned)S.nblk_t1));  // the next slice reads this one's results
+    S.ticket = D->fb_state + 2;
+    if (oax < rank) {
+      const int st[3] = {1, D->GD[0], D->GD[0] * D->GD[1]};
+      S.xch_in_B = D->xch == nullptr;
+      S.xch = S.xch_in_B ? D->B + (long long)(S_VX + oax) * D->cells : D->xch;
+      S.x_c = S.xch_in_B ? st[dim] : 1;
+      S.x_1 = S.xch_in_B ? st[rax] : N;
+      S.x_2 = S.xch_in_B ? st[oax] : N * D->GD[rax];
     }
+  } else {
+    S.ax_t1 = dim == 0 ? 1 : 0;
+    S.ax_t2 = dim == 2 ? 1 : 2;
   }
+  S.n_t1 = D->GD[S.ax_t1];
+  S.n_t2 = D->GD[S.ax_t2];
+  S.t2_0 = 0;
+  set_strides(S);
+  S.nblk_t1 = (S.n_t1 + kTP - 1) / kTP;
+  const long long nblk = (long long)S.nseg * S.nblk_t1 * S.n_t2;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (D->profile && !S.pipe) {
+    if (D->ev_used + 2 > D->ev.size()) {
+      for (int k = 0; k < 2; k++) {
+        hipEvent_t e;
+        HIPCHK(hipEventCreate(&e));
+        D->ev.push_back(e);
+      }
+    }
+    e0 = D->ev[D->ev_used];
+    e1 = D->ev[D->ev_used + 1];
+    D->ev_used += 2;
+    HIPCHK(hipEventRecord(e0, D->stream));
+  }
+  HIPCHK(S.pipe ? launch_tiles((unsigned)nblk, std::integral_constant<int, 1>())
+                : launch_tiles((unsigned)nblk, std::integral_constant<int, 0>()));
+  if (e1) HIPCHK(hipEventRecord(e1, D->stream));
+  HIPCHK(launch_fb((unsigned)(nblk / S.nseg)));
   std::swap(D->A, D->B);
   return ENZO_PPM_SUCCESS;
 }
@@ -832,8 +853,13 @@ int hipPPMInitData(hipPPMData **Data, const hipPPMParameter *Para, void *stream)
     D->fb_groups = ngrp;
     if (alloc_dev((void **)&D->fb_flag, sizeof(int) * ngrp) ||
         alloc_dev((void **)&D->fb_list, sizeof(unsigned) * ngrp) ||
-        alloc_dev((void **)&D->fb_state, 2 * sizeof(unsigned)))
+        alloc_dev((void **)&D->fb_state, 3 * sizeof(unsigned)))
       return ENZO_PPM_ERR_HIP;
+  }
+  if (Para->PPMDiffusionParameter != 0 && !D->xch &&
+      hipMalloc((void **)&D->xch, sizeof(double) * (size_t)cells) != hipSuccess) {
+    (void)hipGetLastError();  // the exchange stays in the state's own arrays
+    D->xch = nullptr;
   }
   D->stream = (hipStream_t)stream;
   // geometry tables and segments (cheap; rebuilt on every init)
@@ -1168,11 +1194,13 @@ int hipPPMSolvePPM_DE_NoAlloc(const enzo_ppm_grid *g, const enzo_ppm_globals *gl
   D.fb_groups = fallback_groups(D.GD);
   D.fb_flag = sc.take<int>((size_t)D.fb_groups);
   D.fb_list = sc.take<unsigned>((size_t)D.fb_groups);
-  D.fb_state = sc.take<unsigned>(2);
+  D.fb_state = sc.take<unsigned>(3);
   static thread_local int segs[2 * 3 * ENZO_PPM_MAX_ANY_SINGLE_DIRECTION];
   const int nsegs = plan_segments(&D, &Para, segs);
   if (nsegs < 0) return ENZO_PPM_ERR_ARGUMENT;
   D.segbuf = sc.take<int>((size_t)std::max(1, nsegs));
+  if (Para.PPMDiffusionParameter != 0 && sc.used + 256 + sizeof(double) * cells <= kScratchBytes)
+    D.xch = sc.take<double>(cells);  // else the exchange stays in the state's own arrays
   if (sc.used > kScratchBytes) {
     snprintf(g_last_error, sizeof(g_last_error),
              "hipPPMSolvePPM_DE_NoAlloc: the grid needs %zu bytes of scratch, more than its "

@@ -118,7 +118,16 @@ using FbCfg = Cfg<1, kFbTS>;
 // error: put the tile's pencil group on the fallback list once (the group
 // flag deduplicates the tiles of one group); the entry carries P.fb_tag
 // (the grid of a batched level, 0 otherwise).
+// Diffusion in one launch: a failing slice changes every later slice of its
+// rows, so the entry is the row group and its flag the first failing slice,
+// as slice - n_t2 (the smallest wins).
 __device__ inline void flag_group(const SweepParams &P, int grp) {
+  if (P.pipe) {
+    const int row = grp % P.nblk_t1, k = grp / P.nblk_t1;
+    if (atomicMin(&P.fb_flag[row], k - P.n_t2) == 0)
+      P.fb_list[atomicAdd(P.fb_count, 1u)] = (unsigned)row;
+    return;
+  }
   if (atomicExch(&P.fb_flag[grp], 1) == 0)
     P.fb_list[atomicAdd(P.fb_count, 1u)] = P.fb_tag + (unsigned)grp;
 }
@@ -138,10 +147,27 @@ __device__ inline void tile_done(const SweepParams &P, int tile, const TileCount
 }
 
 // Every pencil of group `grp` (P.tp pencils along t1) redone whole with the
-// per-cell fallback, then the group flag cleared.
+// per-cell fallback, then the group flag cleared.  Diffusion in one launch
+// (flag_group): the row group's slices from the first failing one on, in
+// order, each reading the one before it.
+template <int UNI, int LEARN = 0, int TS = kFbTS>
+__device__ inline void fallback_pencils(const SweepParams &P, int tb, int t2, double *sm, DevExec &ex);
 template <int UNI, int LEARN = 0, int TS = kFbTS>
 __device__ inline void fallback_group(const SweepParams &P, int grp, double *sm, DevExec &ex) {
-  const int tb = grp % P.nblk_t1, t2 = P.t2_0 + grp / P.nblk_t1;
+  if (P.pipe) {
+    const int first = P.n_t2 + P.fb_flag[grp];
+    for (int k = first; k < P.n_t2; k++) {
+      fallback_pencils<UNI, LEARN, TS>(P, grp, k, sm, ex);
+      __threadfence();
+      __syncthreads();
+    }
+  } else {
+    fallback_pencils<UNI, LEARN, TS>(P, grp % P.nblk_t1, P.t2_0 + grp / P.nblk_t1, sm, ex);
+  }
+  if (threadIdx.x == 0) P.fb_flag[grp] = 0;
+}
+template <int UNI, int LEARN, int TS>
+__device__ inline void fallback_pencils(const SweepParams &P, int tb, int t2, double *sm, DevExec &ex) {
   for (int p = 0; p < P.tp && tb * P.tp + p < P.n_t1; p++) {
     if (!P.fb_ok) {
       if (threadIdx.x == 0) atomicAdd(&P.counters[3], 1ull);
@@ -154,7 +180,6 @@ __device__ inline void fallback_group(const SweepParams &P, int grp, double *sm,
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) P.fb_flag[grp] = 0;
 }
 
 // Whether a fallback launch has nothing to do.  Every workgroup of a launch
@@ -541,6 +566,7 @@ __device__ inline void fluxcorr_side(const FluxCorrParams &F, long long x, int s
 // the slice (inteuler.F:241-289), so one coefficient row per slice is all the
 // sweep needs.  Items: N + (i2 - i1 + 3) * n_outer.
 __device__ inline void prep_item(const FlatParams &F, long long gid) {
+  if (gid == 0 && F.ticket) *F.ticket = 0u;
   if (gid < F.N) {
     const double dt = F.dtp ? *as_global(F.dtp) : F.dt;
     as_global(F.qc)[gid] = dt / as_global(F.dx)[gid];

@@ -133,6 +133,13 @@ struct SweepParams {
                     // flux_hll fallback (Grid_xEulerSweep.C:258-269); without
                     // it tiles of SV = 1 take flux_hll's fluxes (:245-256)
   int tp;           // pencils per group (the sweep tile's TP)
+  // diffusion in one launch (tiles of DF = 1): the slices' tiles take their
+  // turn from `ticket` and wait for each other's velocities (wait_pair)
+  int pipe;
+  unsigned *ticket;
+  double *xch;            // published velocities (exchange_index), or B's own
+  int x_c, x_1, x_2;      // slot; strides of cell, row and slice; whether it is
+  int xch_in_B;           // B's slot
   // learned two-shock start: network parameters (ppm_learn.hpp), read by
   // the LEARN instantiation only
   const float *learn;
@@ -864,10 +871,99 @@ PPM_HD void harvest_record(const SweepParams &P, int t1, int t2, int i, const do
   for (int m = 0; m < kHarvestDoubles; m++) as_global(P.harvest)[k * kHarvestDoubles + m] = v[m];
 }
 
+// Diffusion in one launch.  The reference's calcdiss reads the transverse
+// velocities of the live state, so slice k needs the velocity along the
+// outer axis that slice k-1 ends with, at the same row: a chain over the
+// slices of each row.  A slice is far too little work for the chip and one
+// launch per slice costs a launch, an empty fallback launch and a tile's
+// whole latency per link (64^3: 24 us, 210 of them per step).  Instead all
+// slices' tiles run in one launch, in slice order (`ticket`); each does
+// everything up to its Godunov states, then waits for the two values of
+// slice k-1 it needs, and publishes its own new values as soon as it has its
+// fluxes.  The message is the value itself: the exchange array is filled
+// with kUnpublished before the launch, values are stored and polled with
+// relaxed 64-bit atomics at agent scope (the tiles of a row run on any XCD),
+// and no other data is passed.  Tiles only ever wait for tiles with an
+// earlier ticket, which run or have run, so the earliest unfinished tile
+// always can finish.  The exchange array holds a row's cells side by side, so
+// that a wavefront polls and stores whole lines; where there is no memory for
+// it, it is the destination's own slot of that velocity, with the grid's
+// strides (64^3: y and z sweeps 340 us instead of 150).  A link of the
+// chain takes about 1.9 us, most of it the two trips through memory.
+// 64^3 Sod step: 4.43 ms with one launch per slice, 0.49 ms.
+constexpr unsigned long long kUnpublished = 0x7ff8dead5eedc0deull;  // a NaN no operation makes
+constexpr int kSpinLimit = 1 << 20;  // polls before a wait gives up (counted as an error)
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// both values once published, spinning meanwhile
+PPM_HD bool wait_pair(const double *pa, bool wa, const double *pb, bool wb, double &a, double &b) {
+  const auto qa = (const unsigned long long PPM_GLOBAL *)pa;
+  const auto qb = (const unsigned long long PPM_GLOBAL *)pb;
+  unsigned long long va = 0, vb = 0;
+  int n = 0;
+  for (; n < kSpinLimit; n++) {
+    va = __hip_atomic_load(qa, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    vb = __hip_atomic_load(qb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!(wa && va == kUnpublished) && !(wb && vb == kUnpublished)) break;
+    __builtin_amdgcn_s_sleep(2);
+  }
+  a = __longlong_as_double((long long)va);
+  b = __longlong_as_double((long long)vb);
+  return n < kSpinLimit;
+}
+PPM_HD void publish(double *p, double v) {
+  unsigned long long x = (unsigned long long)__double_as_longlong(v);
+  if (x == kUnpublished) x ^= 1ull;  // another payload of the same NaN
+  __hip_atomic_store((unsigned long long PPM_GLOBAL *)p, x, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+// x computed before anything that follows (a wait must not delay it)
+#define PPM_PIN(x) asm volatile("" : "+v"(x))
+#else
+PPM_HD bool wait_pair(const double *pa, bool, const double *pb, bool, double &a, double &b) {
+  a = *pa;  // workgroups run one after the other there, in ticket order
+  b = *pb;
+  return true;
+}
+PPM_HD void publish(double *p, double v) { *p = v; }
+#define PPM_PIN(x) ((void)(x))
+#endif
+
+// Whether a pencil's interfaces are one wavefront's lanes: the Riemann phase
+// then takes the right interface's fluxes from the next lane and publishes at
+// once, ahead of the flux stores and a barrier.  (Work-items run one by one in
+// the CPU execution, which publishes in ph_check.)
+#if defined(__HIP_DEVICE_COMPILE__)
+template <int TS>
+constexpr bool kWavePencil = TS == 64;
+#define PPM_NEXT_LANE(x) __shfl_down((x), 1, 64)
+#else
+template <int TS>
+constexpr bool kWavePencil = false;
+#define PPM_NEXT_LANE(x) (x)
+#endif
+
+// where the velocity of `cell` (1-based) of a slice's row is published
+PPM_HD long long exchange_index(const SweepParams &P, int row, int slice, int cell) {
+  return (long long)(cell - 1) * P.x_c + (long long)row * P.x_1 + (long long)slice * P.x_2;
+}
+
+// The new velocity w along the outer axis (ph_euler's expressions) of a cell
+// with density d and old velocity w, its left and right interfaces' fluxes
+// given, published for the next slice.
+PPM_HD void publish_velocity(const SweepParams &P, int t1, int t2, int cell, double d, double w,
+                             double dfl, double dfr, double wfl, double wfr) {
+  double dnu = d + (dfl - dfr);
+  if (P.dfloor > 0.0) dnu = fmx(dnu, P.dfloor);
+  publish(P.xch + exchange_index(P, t1, t2, cell), (w * d + (wfl - wfr)) * (1.0 / dnu));
+}
+
 // diffusion coefficient at interface i (calcdiss.F:207-236, 377-404);
 // transverse velocities come from the 3-D state: the current slice and the
 // next one from A, the previous slice (already swept) from B.
-template <int TP, int TS, int UNI = 0>
+// PIPE: the previous slice's tile may still be running (wait_pair); cells
+// outside [i1, i2] keep their velocities, so A holds them too.
+template <int TP, int TS, int UNI = 0, int PIPE = 0>
 PPM_HD double diffcoef1(const SweepParams &P, const Tile &T, double *sm, int p, int i) {
   const int rax = (P.dim + 1) % 3, oax = (P.dim + 2) % 3;
   const int t1 = T.t1_0 + p, t2 = T.t2;
@@ -890,11 +986,27 @@ PPM_HD double diffcoef1(const SweepParams &P, const Tile &T, double *sm, int p, 
     dc = dc + (TS_<UNI>(P, T_DIFFX, i) / TR_(P, T_DDEN, j, jdim)) * vdiff1;
   }
   if (P.nact_out > 1 && 1 < k && k < kdim) {  // nzz > 1 .and. lk1 (dimz > 1 .and. lkz1)
-    const auto wo = as_global(P.A) + (long long)(S_VX + oax) * P.cells;
-    const auto wn = as_global(P.B) + (long long)(S_VX + oax) * P.cells;
-    double wdiff1 = (wn[at(row, outer - 1, i)] + wn[at(row, outer - 1, i - 1)]) -
-                    (wo[at(row, outer + 1, i)] + wo[at(row, outer + 1, i - 1)]);
-    dc = dc + (TS_<UNI>(P, T_DIFFX, i) / TO_(P, T_DDEN, k, kdim)) * wdiff1;
+    const long long slot = (long long)(S_VX + oax) * P.cells;
+    const auto wo = as_global(P.A) + slot;
+    double old2 = wo[at(row, outer + 1, i)] + wo[at(row, outer + 1, i - 1)];
+    double ratio = TS_<UNI>(P, T_DIFFX, i) / TO_(P, T_DDEN, k, kdim);
+    double n0, n1;
+    if constexpr (PIPE != 0) {
+      const bool b0 = i <= P.i2, b1 = i - 1 >= P.i1;
+      const double *q0 = b0 ? P.xch + exchange_index(P, row, outer - 1, i) : P.A + slot + at(row, outer - 1, i);
+      const double *q1 = b1 ? P.xch + exchange_index(P, row, outer - 1, i - 1)
+                            : P.A + slot + at(row, outer - 1, i - 1);
+      PPM_PIN(dc);
+      PPM_PIN(old2);
+      PPM_PIN(ratio);
+      if (!wait_pair(q0, b0, q1, b1, n0, n1)) PPM_ATOMIC_ADD_U64(&P.counters[2], 1);
+    } else {
+      const auto wn = as_global(P.B) + slot;
+      n0 = wn[at(row, outer - 1, i)];
+      n1 = wn[at(row, outer - 1, i - 1)];
+    }
+    double wdiff1 = (n0 + n1) - old2;
+    dc = dc + ratio * wdiff1;
   }
   return 0.1 * fmx(0.0, dc);
 }
@@ -1030,11 +1142,11 @@ PPM_HD void hllc_flux(const HllIn &h, Regs &r) {
 
 // the diffusion terms of an interface's HLL / HLLC fluxes (flux_hll.F:166-195)
 // from its diffusion coefficient dc
-template <int TP, int TS, int UNI = 0>
+template <int TP, int TS, int UNI = 0, int DF = -1>
 PPM_HD void hll_diffusion(const SweepParams &P, const Tile &T, double *sm, int p, int i, double dc,
                           HllIn &h) {
   h.diffd = h.diffuu = h.diffuv = h.diffuw = h.diffue = h.diffuge = 0.0;
-  if (P.idiff == 0) return;
+  if (!(DF < 0 ? P.idiff != 0 : DF != 0)) return;
   const int ca = i - 1 - T.L0, cb = i - T.L0;
   const double da = LDS<TP, TS, UNI>(sm, A_D, p, ca), dbb = LDS<TP, TS, UNI>(sm, A_D, p, cb);
   h.diffd = dc * (da - dbb);
@@ -1054,7 +1166,21 @@ PPM_HD void hll_diffusion(const SweepParams &P, const Tile &T, double *sm, int p
 // STAGE 1 continues from them (with Regs::ls / lc, the interface's network
 // correction).
 // SV 0: the two-shock solver; 1: HLL or HLLC (P.hllc) fluxes in its place.
-template <int TP, int TS, int UNI = 0, int FB = 0, int LEARN = 0, int STAGE = 2, int SV = 0>
+// DF 0: no diffusion; 1: diffusion in one launch (wait_pair); -1: P.idiff,
+// the slices in order.
+template <int DF>
+PPM_HD bool diffusion_on(const SweepParams &P) {
+  return DF < 0 ? P.idiff != 0 : DF != 0;
+}
+template <int TP, int TS, int UNI = 0>
+PPM_HD void ph_publish(const SweepParams &P, const Tile &T, double *sm, int p, int i, const Regs &r) {
+  const double dfr = PPM_NEXT_LANE(r.df), wfr = PPM_NEXT_LANE(r.wf);
+  if (!P.xch || i < T.o || i >= T.o + T.w || i < P.i1 || i > P.i2) return;
+  const int c = i - T.L0;
+  publish_velocity(P, T.t1_0 + p, T.t2, i, LDS<TP, TS, UNI>(sm, A_D, p, c),
+                   LDS<TP, TS, UNI>(sm, A_W, p, c), r.df, dfr, r.wf, wfr);
+}
+template <int TP, int TS, int UNI = 0, int FB = 0, int LEARN = 0, int STAGE = 2, int SV = 0, int DF = -1>
 PPM_HD void ph_solve(const SweepParams &P, const Tile &T, double *sm, int tid, Regs &r) {
   int p = tid / TS, q = tid % TS;
   if constexpr (FB != 0 && STAGE != 1) r.hll = 0;
@@ -1169,8 +1295,9 @@ PPM_HD void ph_solve(const SweepParams &P, const Tile &T, double *sm, int tid, R
     HllIn h;
     h.dls = dls; h.drs = drs; h.pls = pls; h.prs = prs; h.uls = uls; h.urs = urs;
     h.vls = r.vls; h.vrs = r.vrs; h.wls = r.wls; h.wrs = r.wrs; h.gels = r.gels; h.gers = r.gers;
-    hll_diffusion<TP, TS, UNI>(
-        P, T, sm, p, i, P.idiff != 0 ? diffcoef1<TP, TS, UNI>(P, T, sm, p, i) : 0.0, h);
+    hll_diffusion<TP, TS, UNI, DF>(
+        P, T, sm, p, i,
+        diffusion_on<DF>(P) ? diffcoef1<TP, TS, UNI, DF == 1>(P, T, sm, p, i) : 0.0, h);
     h.gamma = gamma;
     h.qc = qc_of<UNI>(P, T, i);
     h.idual = P.idual;
@@ -1184,6 +1311,7 @@ PPM_HD void ph_solve(const SweepParams &P, const Tile &T, double *sm, int tid, R
       r.c_ga = r.h_sl * r.h_bm0;
       r.c_gb = r.h_sr * r.h_bp0;
     }
+    if constexpr (DF == 1 && kWavePencil<TS>) ph_publish<TP, TS, UNI>(P, T, sm, p, i, r);
     return;
   }
   // two-shock solution
@@ -1240,8 +1368,14 @@ PPM_HD void ph_solve(const SweepParams &P, const Tile &T, double *sm, int tid, R
   double dub = ub * db;
   double duub, duvb, duwb, dueb, dugeb = 0.0;
   double dc = 0.0;
-  if (P.idiff != 0) {  // flux_twoshock.F:291-322
-    dc = diffcoef1<TP, TS, UNI>(P, T, sm, p, i);
+  if (diffusion_on<DF>(P)) {  // flux_twoshock.F:291-322
+    if constexpr (DF == 1) {
+      PPM_PIN(dub);
+      PPM_PIN(vb);
+      PPM_PIN(wb);
+      PPM_PIN(eb);
+    }
+    dc = diffcoef1<TP, TS, UNI, DF == 1>(P, T, sm, p, i);
     double da = LDS<TP, TS, UNI>(sm, A_D, p, ca), dbb = LDS<TP, TS, UNI>(sm, A_D, p, cb);
     duub = dub * ub + dc * (da * LDS<TP, TS, UNI>(sm, A_U, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_U, p, cb));
     duvb = dub * vb + dc * (da * LDS<TP, TS, UNI>(sm, A_V, p, ca) - dbb * LDS<TP, TS, UNI>(sm, A_V, p, cb));
@@ -1265,6 +1399,7 @@ PPM_HD void ph_solve(const SweepParams &P, const Tile &T, double *sm, int tid, R
   r.vf = qc * duvb;
   r.wf = qc * duwb;
   r.gef = qc * dugeb;
+  if constexpr (DF == 1 && kWavePencil<TS>) ph_publish<TP, TS, UNI>(P, T, sm, p, i, r);
   r.ub = ub;
   r.db = db;
   if constexpr (FB != 0) {
@@ -1347,7 +1482,8 @@ PPM_HD void upd_range(const SweepParams &P, const Tile &T, int &c0, int &c1) {
 // Phase: negative density / energy check (flux_twoshock.F:401-403; the HLL
 // and HLLC solvers check the density alone, flux_hll.F:349-351 and
 // flux_hllc.F:344).  Returns the number of failing cells seen by this thread.
-template <int TP, int TS, int UNI = 0, int SV = 0>
+// DF 1: also publishes the owned cells' velocities, unless ph_solve did.
+template <int TP, int TS, int UNI = 0, int SV = 0, int DF = -1>
 PPM_HD int ph_check(const SweepParams &P, const Tile &T, double *sm, int tid) {
   int c0, c1;
   upd_range(P, T, c0, c1);
@@ -1359,6 +1495,10 @@ PPM_HD int ph_check(const SweepParams &P, const Tile &T, double *sm, int tid) {
     int c = cell - T.L0;
     double d = LDS<TP, TS, UNI>(sm, A_D, p, c), e = LDS<TP, TS, UNI>(sm, A_E, p, c);
     double dfl = LDS<TP, TS, UNI>(sm, F_DF, p, c), dfr = LDS<TP, TS, UNI>(sm, F_DF, p, c + 1);
+    if constexpr (DF == 1 && !kWavePencil<TS>)
+      if (P.xch && cell >= T.o && cell < T.o + T.w)
+        publish_velocity(P, T.t1_0 + p, T.t2, cell, d, LDS<TP, TS, UNI>(sm, A_W, p, c), dfl, dfr,
+                         LDS<TP, TS, UNI>(sm, F_WF, p, c), LDS<TP, TS, UNI>(sm, F_WF, p, c + 1));
     if (SV != 0 ? (d + dfl) - dfr <= 0.0 : (d + (dfl - dfr) <= 0.0 || e < 0.0)) bad++;
   }
   return bad;
@@ -1541,7 +1681,7 @@ PPM_HD void ph_pgas_spec(const SweepParams &P, const Tile &T, double *sm, int ti
 // write every owned cell of the hydro fields to B.  The speculative e is
 // exact unless the demax test changed ge in a cell whose e uses ge (never
 // with positive energies); those cells are recomputed here and counted.
-template <int TP, int TS, int UNI = 0>
+template <int TP, int TS, int UNI = 0, int DF = -1>
 PPM_HD int ph_pgas_write(const SweepParams &P, const Tile &T, double *sm, int tid) {
   int g0, g1;
   pg_range(P, g0, g1);
@@ -1582,7 +1722,9 @@ PPM_HD int ph_pgas_write(const SweepParams &P, const Tile &T, double *sm, int ti
     B[S_E * P.cells + g] = e;
     B[(S_VX + P.dim) * P.cells + g] = u;
     B[(S_VX + vax) * P.cells + g] = vax < P.rank ? v : A[(S_VX + vax) * P.cells + g];
-    B[(S_VX + wax) * P.cells + g] = wax < P.rank ? w : A[(S_VX + wax) * P.cells + g];
+    // (an exchange in B's slot has the updated cells' w already)
+    if (DF != 1 || !P.xch_in_B || cell < P.i1 || cell > P.i2)
+      B[(S_VX + wax) * P.cells + g] = wax < P.rank ? w : A[(S_VX + wax) * P.cells + g];
     if (P.idual) B[S_GE * P.cells + g] = ge;
   });
   return chains;
@@ -1714,6 +1856,10 @@ struct FlatParams {
   double dt;
   const double *dtp;  // device dt if non-null
   double *qc;         // out: dt/dx(i), i = 1..N
+  // diffusion in one launch: what to fill with kUnpublished and the ticket to
+  // set to 0 (null otherwise)
+  double *unpublished;  // the exchange array, `cells` doubles
+  unsigned *ticket;
 };
 
 PPM_HD double flat_value(const FlatParams &F, int outer, int cell) {
@@ -1923,7 +2069,7 @@ PPM_HD void sweep_var(const SweepParams &P, const Tile &T, double *sm, X &ex) {
   ex.run([&](int tid, Regs &r) { ph_iface<V, TP, TS, UNI>(P, T, sm, tid, r); });
 }
 
-template <int TP, int TS, int UNI, int FB, class X, int LEARN = 0, int SV = 0>
+template <int TP, int TS, int UNI, int FB, class X, int LEARN = 0, int SV = 0, int DF = -1>
 PPM_HD TileCounts sweep_body(const SweepParams &P, const Tile &T, double *sm, X &ex) {
   TileCounts tc;
   tc.nfb = 0;
@@ -1950,12 +2096,12 @@ PPM_HD TileCounts sweep_body(const SweepParams &P, const Tile &T, double *sm, X 
     const int m = *NetLds<TP, TS, UNI>::count(sm);  // the same for every work-item
     if (m > 0) learn_eval<TP, TS, UNI>(P, sm, m, ex);
     ex.run([&](int tid, Regs &r) {
-      ph_solve<TP, TS, UNI, FB, LEARN, 1>(P, T, sm, tid, r);
+      ph_solve<TP, TS, UNI, FB, LEARN, 1, 0, DF>(P, T, sm, tid, r);
       ph_store_flux<TP, TS, UNI, FB>(P, T, sm, tid, r);
     });
   } else {
     ex.run([&](int tid, Regs &r) {
-      ph_solve<TP, TS, UNI, FB, LEARN, 2, SV>(P, T, sm, tid, r);
+      ph_solve<TP, TS, UNI, FB, LEARN, 2, SV, DF>(P, T, sm, tid, r);
       ph_store_flux<TP, TS, UNI, FB, SV>(P, T, sm, tid, r);
     });
   }
@@ -1965,7 +2111,7 @@ PPM_HD TileCounts sweep_body(const SweepParams &P, const Tile &T, double *sm, X 
       ex.run([&](int tid, Regs &r) { ph_hllc_ges_store<TP, TS, UNI>(P, T, sm, tid, r); });
     }
   }
-  tc.bad = ex.count([&](int tid, Regs &r) { (void)r; return ph_check<TP, TS, UNI, SV>(P, T, sm, tid); });
+  tc.bad = ex.count([&](int tid, Regs &r) { (void)r; return ph_check<TP, TS, UNI, SV, DF>(P, T, sm, tid); });
   bool fbon = false;
   int fberr = 0;
   if constexpr (FB != 0) {
@@ -1988,7 +2134,7 @@ PPM_HD TileCounts sweep_body(const SweepParams &P, const Tile &T, double *sm, X 
   tc.err += fberr;
   if (P.idual) ex.run([&](int tid, Regs &r) { (void)r; ph_pgas_spec<TP, TS, UNI>(P, T, sm, tid); });
   tc.chains =
-      ex.count([&](int tid, Regs &r) { (void)r; return ph_pgas_write<TP, TS, UNI>(P, T, sm, tid); });
+      ex.count([&](int tid, Regs &r) { (void)r; return ph_pgas_write<TP, TS, UNI, DF>(P, T, sm, tid); });
   for (int n = 0; n < P.ncol; n++) {
     ex.run([&](int tid, Regs &r) { (void)r; ph_load_col<TP, TS, UNI>(P, T, sm, tid, n); });
     ex.run([&](int tid, Regs &r) { (void)r; ph_slope<TP, TS, UNI>(P, T, sm, tid, A_COL); });
@@ -2010,9 +2156,9 @@ PPM_HD TileCounts sweep_body(const SweepParams &P, const Tile &T, double *sm, X 
 // workgroup per pencil, which held it whole and solved the two-shock problem
 // first: 1,310 us), at 160^3 with two colours the HLLC sweep 510 us
 // (3,980 us).
-template <int TP, int TS, int UNI, class X, int LEARN = 0, int SV = 0>
+template <int TP, int TS, int UNI, class X, int LEARN = 0, int SV = 0, int DF = -1>
 PPM_HD TileCounts sweep_tile(const SweepParams &P, int block, double *sm, X &ex) {
-  return sweep_body<TP, TS, UNI, 0, X, LEARN, SV>(P, make_tile<TP, TS, UNI>(P, block), sm, ex);
+  return sweep_body<TP, TS, UNI, 0, X, LEARN, SV, DF>(P, make_tile<TP, TS, UNI>(P, block), sm, ex);
 }
 
 // One whole pencil in a one-pencil workgroup of TS threads, with the
