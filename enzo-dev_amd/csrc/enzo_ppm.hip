@@ -37,12 +37,13 @@ using SweepCfg = Cfg<kTP, kTS>;
 // DF 1: diffusion in one launch (wait_pair).  DF 0 keeps the tile's test of
 // P.idiff, never set there: it splits the Riemann phase, which the compiler
 // then schedules better (256^3 step 7.50 ms; 7.70 without the test).
-template <int UNI, int LEARN, int SV, int DF>
+template <int UNI, int LEARN, int SV, int DF, int FAST>
 // 5 wavefronts per SIMD: 96 VGPRs (a few spilled) and 31 KB of LDS per
 // workgroup, 5 workgroups per CU.  The HLL / HLLC tile (SV) keeps more
 // interface values live: 4 wavefronts (116 VGPRs, 6 spilled) take 1.64 ms
-// per 160^3 HLLC step against 1.89 ms with 5 (24 spilled).
-__global__ __launch_bounds__(kTP *kTS) __attribute__((amdgpu_waves_per_eu((SV == 0 ? 5 : 4))))
+// per 160^3 HLLC step against 1.89 ms with 5 (24 spilled).  So do the fast
+// tiles (FAST; 110 VGPRs): 6.61 ms per 256^3 step, 7.16 with 5 (14 spilled).
+__global__ __launch_bounds__(kTP *kTS) __attribute__((amdgpu_waves_per_eu((SV == 0 && FAST == 0 ? 5 : 4))))
 void ppm_sweep_kernel(SweepParams P) {
   __shared__ double sm[SweepCfg::SMEM];
   PPM_LDS_ENTER(sm);
@@ -56,7 +57,9 @@ void ppm_sweep_kernel(SweepParams P) {
     __syncthreads();
     tile = PPM_UNIFORM(turn);
   }
-  tile_done<SV>(P, tile, sweep_tile<kTP, kTS, UNI, DevExec, LEARN, SV, DF == 0 ? -1 : DF>(P, tile, sm, ex));
+  const TileCounts tc =
+      sweep_tile<kTP, kTS, UNI, DevExec, LEARN, SV, DF == 0 ? -1 : DF, FAST>(P, tile, sm, ex);
+  tile_done<SV, FAST>(P, tile, tc, ex);
 }
 
 // ------------------------------------------------------------------------
@@ -561,19 +564,24 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
   // with the HLL and HLLC solvers, which have no use for the learned start
   const int variant = (S.uni[0] ? 1 : 0) | (D->learned ? 2 : 0);
   const bool two_shock = P->RiemannSolver == ENZO_PPM_RIEMANN_TWOSHOCK;
+  const bool fast = set_fast(S) && two_shock && !D->learned && D->harvest_cap == 0;
   auto launch_tiles = [&](unsigned nblk, auto diff) {
     constexpr int DF = decltype(diff)::value;
     const dim3 g(nblk), b(kTP * kTS);
     if (!two_shock) {
-      if (S.uni[0]) hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 1, DF>), g, b, 0, D->stream, S);
-      else hipLaunchKernelGGL((ppm_sweep_kernel<0, 0, 1, DF>), g, b, 0, D->stream, S);
+      if (S.uni[0]) hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 1, DF, 0>), g, b, 0, D->stream, S);
+      else hipLaunchKernelGGL((ppm_sweep_kernel<0, 0, 1, DF, 0>), g, b, 0, D->stream, S);
+      return hipGetLastError();
+    }
+    if (fast) {
+      hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 0, DF, 1>), g, b, 0, D->stream, S);
       return hipGetLastError();
     }
     switch (variant) {
-      case 0: hipLaunchKernelGGL((ppm_sweep_kernel<0, 0, 0, DF>), g, b, 0, D->stream, S); break;
-      case 1: hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 0, DF>), g, b, 0, D->stream, S); break;
-      case 2: hipLaunchKernelGGL((ppm_sweep_kernel<0, 1, 0, DF>), g, b, 0, D->stream, S); break;
-      default: hipLaunchKernelGGL((ppm_sweep_kernel<1, 1, 0, DF>), g, b, 0, D->stream, S); break;
+      case 0: hipLaunchKernelGGL((ppm_sweep_kernel<0, 0, 0, DF, 0>), g, b, 0, D->stream, S); break;
+      case 1: hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 0, DF, 0>), g, b, 0, D->stream, S); break;
+      case 2: hipLaunchKernelGGL((ppm_sweep_kernel<0, 1, 0, DF, 0>), g, b, 0, D->stream, S); break;
+      default: hipLaunchKernelGGL((ppm_sweep_kernel<1, 1, 0, DF, 0>), g, b, 0, D->stream, S); break;
     }
     return hipGetLastError();
   };

@@ -136,8 +136,12 @@ __device__ inline void flag_group(const SweepParams &P, int grp) {
 // group on the fallback list, which redoes the group's pencils whole (the
 // fallback chain can cross segments) and settles them; with the HLL solver
 // there is no fallback and either is an error.
-template <int SV>
-__device__ inline void tile_done(const SweepParams &P, int tile, const TileCounts &tc) {
+// FAST: an operand out of range (Regs::oob) does the same.
+template <int SV, int FAST = 0>
+__device__ inline void tile_done(const SweepParams &P, int tile, const TileCounts &tc,
+                                 const DevExec &ex) {
+  if constexpr (FAST != 0)
+    if (ex.r.oob) flag_group(P, tile / P.nseg);
   if (threadIdx.x != 0) return;
   if (tc.bad || tc.err) {
     if (SV == 0 || P.hllc) flag_group(P, tile / P.nseg);

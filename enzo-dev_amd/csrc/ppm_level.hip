@@ -58,15 +58,16 @@ constexpr int kShapes = 3;
 constexpr int kShapeTP[kShapes] = {16, 8, 4};
 constexpr int kShapeTS[kShapes] = {16, 32, 64};
 
-template <int TP, int TS, int UNI, int LEARN, int SV>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((SV == 0 ? 5 : 4))))
+template <int TP, int TS, int UNI, int LEARN, int SV, int FAST>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((SV == 0 && FAST == 0 ? 5 : 4))))
 void level_sweep_kernel(const SweepParams *__restrict__ params, const Work *__restrict__ work) {
   __shared__ double sm[Cfg<TP, TS>::SMEM];
   PPM_LDS_ENTER(sm);
   DevExec ex;
   const Work w = work[xcd_tile((int)blockIdx.x, (int)gridDim.x)];
   const SweepParams &P = params[w.grid];
-  tile_done<SV>(P, w.tile, sweep_tile<TP, TS, UNI, DevExec, LEARN, SV>(P, w.tile, sm, ex));
+  const TileCounts tc = sweep_tile<TP, TS, UNI, DevExec, LEARN, SV, -1, FAST>(P, w.tile, sm, ex);
+  tile_done<SV, FAST>(P, w.tile, tc, ex);
 }
 
 // The same sweep as one persistent launch: a few workgroups per CU, each
@@ -78,7 +79,7 @@ void level_sweep_kernel(const SweepParams *__restrict__ params, const Work *__re
 // finished, and the last of them puts both back to 0 for the next launch
 // (graph replays included).  Every workgroup leaves the loop once its pull
 // passes its range's end, so every item is taken exactly once.
-template <int TP, int TS, int UNI, int LEARN>
+template <int TP, int TS, int UNI, int LEARN, int FAST>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void level_sweep_persistent_kernel(const SweepParams *__restrict__ params,
                                    const Work *__restrict__ work, int nitems, unsigned *queue) {
@@ -104,7 +105,8 @@ void level_sweep_persistent_kernel(const SweepParams *__restrict__ params,
     // compiler hoists every tid-derived address of the tile out of the loop
     // and keeps them all live (spilling registers)
     PPM_OPAQUE_VGPR(ex.tid);
-    tile_done<0>(P, w.tile, sweep_tile<TP, TS, UNI, DevExec, LEARN>(P, w.tile, sm, ex));
+    const TileCounts tc = sweep_tile<TP, TS, UNI, DevExec, LEARN, 0, -1, FAST>(P, w.tile, sm, ex);
+    tile_done<0, FAST>(P, w.tile, tc, ex);
   }
   if (threadIdx.x == 0) {
     const unsigned nx = gridDim.x / nparts + ((int)(gridDim.x % nparts) > x ? 1u : 0u);
@@ -313,6 +315,8 @@ struct hipPPMLevel {
   FlatParams *dflat = nullptr;      // [parity 2][axis 3][grid]
   PresParams *dpres = nullptr;      // [parity 2][grid]
   Work *dwork = nullptr;            // all work lists
+  // every grid with one cell width along the axis may take the fast tiles
+  bool fast[3] = {false, false, false};
   int fb_ts[3] = {kFbTS, kFbTS, kFbTS};  // workgroup width holding every grid's pencils
   Work *dpwork = nullptr;           // pressure chunks
   long long npwork = 0;
@@ -552,6 +556,7 @@ int build_plan(hipPPMLevel *L) {
   }
   for (int d = 0; d < L->rank; d++) {
     // parameters of every grid for axis d
+    L->fast[d] = true;
     int max_slices = 1;
     for (int g = 0; g < G; g++) {
       const int *gd = &L->GD[3 * g];
@@ -624,6 +629,7 @@ int build_plan(hipPPMLevel *L) {
         S.fb_tag = (unsigned)L->grp_off[g];
         S.fb_ok = pencil_fits<kFbTS>(S) ? 1 : 0;
         S.hllc = P0.RiemannSolver == ENZO_PPM_RIEMANN_HLLC ? 1 : 0;
+        if (!set_fast(S) && S.uni[0]) L->fast[d] = false;
         FlatParams &F = hflat[((size_t)par * 3 + d) * G + g];
         memset(&F, 0, sizeof(F));
         F.dim = d;
@@ -755,20 +761,22 @@ int launch_level_sweep(hipPPMLevel *L, int d) {
       unsigned *queue = L->queues + (size_t)2 * kXCD * ln.queue;
       const int nit = (int)ln.count;
       // HLL and HLLC have no persistent form and no use for the learned start
-#define LEVEL_LAUNCH1(TP, TS, U, LRN)                                                         \
+#define LEVEL_LAUNCH1(TP, TS, U, LRN, FST)                                                    \
   if (!two_shock)                                                                           \
-    hipLaunchKernelGGL((level_sweep_kernel<TP, TS, U, 0, 1>), grid, blk, 0, L->stream, P, w); \
+    hipLaunchKernelGGL((level_sweep_kernel<TP, TS, U, 0, 1, 0>), grid, blk, 0, L->stream, P, w); \
   else if (L->persistent)                                                                   \
-    hipLaunchKernelGGL((level_sweep_persistent_kernel<TP, TS, U, LRN>), pgrid, blk, 0,       \
+    hipLaunchKernelGGL((level_sweep_persistent_kernel<TP, TS, U, LRN, FST>), pgrid, blk, 0,  \
                        L->stream, P, w, nit, queue);                                         \
   else                                                                                      \
-    hipLaunchKernelGGL((level_sweep_kernel<TP, TS, U, LRN, 0>), grid, blk, 0, L->stream, P, w);
+    hipLaunchKernelGGL((level_sweep_kernel<TP, TS, U, LRN, 0, FST>), grid, blk, 0, L->stream, P, w);
 #define LEVEL_LAUNCH(S, TP, TS)                                                             \
   if (ln.shape == S) {                                                                    \
     if (L->learned) {                                                                     \
-      if (ln.uni) { LEVEL_LAUNCH1(TP, TS, 1, 1) } else { LEVEL_LAUNCH1(TP, TS, 0, 1) }   \
+      if (ln.uni) { LEVEL_LAUNCH1(TP, TS, 1, 1, 0) } else { LEVEL_LAUNCH1(TP, TS, 0, 1, 0) } \
+    } else if (ln.uni) {                                                                  \
+      if (L->fast[d]) { LEVEL_LAUNCH1(TP, TS, 1, 0, 1) } else { LEVEL_LAUNCH1(TP, TS, 1, 0, 0) } \
     } else {                                                                              \
-      if (ln.uni) { LEVEL_LAUNCH1(TP, TS, 1, 0) } else { LEVEL_LAUNCH1(TP, TS, 0, 0) }   \
+      LEVEL_LAUNCH1(TP, TS, 0, 0, 0)                                                      \
     }                                                                                     \
   }
       LEVEL_LAUNCH(0, 16, 16)
@@ -1362,6 +1370,8 @@ int hipPPMLevelSetExpansionFactors(hipPPMLevel *L, enzo_float a_courant, enzo_fl
           S.kt_out[t] = L->kt[((size_t)3 * g + oax) * NTAB + t];
         }
         set_dx_inverse(S);
+        // the widths left the fast tiles' range: another kernel, other graphs
+        if (!set_fast(S) && S.uni[0] && L->fast[d]) return build_plan(L);
       }
   LCHK(hipMemcpy(L->dparams, L->hparams.data(), sizeof(SweepParams) * L->hparams.size(),
                  hipMemcpyHostToDevice));
