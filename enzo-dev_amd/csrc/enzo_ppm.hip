@@ -42,7 +42,7 @@ template <int UNI, int LEARN, int SV, int DF, int FAST>
 // workgroup, 5 workgroups per CU.  The HLL / HLLC tile (SV) keeps more
 // interface values live: 4 wavefronts (116 VGPRs, 6 spilled) take 1.64 ms
 // per 160^3 HLLC step against 1.89 ms with 5 (24 spilled).  So do the fast
-// tiles (FAST; 110 VGPRs): 6.61 ms per 256^3 step, 7.16 with 5 (14 spilled).
+// tiles (FAST; 110 VGPRs): 6.2 ms per 256^3 step, 6.65 with 5 (10 spilled).
 __global__ __launch_bounds__(kTP *kTS) __attribute__((amdgpu_waves_per_eu((SV == 0 && FAST == 0 ? 5 : 4))))
 void ppm_sweep_kernel(SweepParams P) {
   __shared__ double sm[SweepCfg::SMEM];
@@ -59,7 +59,7 @@ void ppm_sweep_kernel(SweepParams P) {
   }
   const TileCounts tc =
       sweep_tile<kTP, kTS, UNI, DevExec, LEARN, SV, DF == 0 ? -1 : DF, FAST>(P, tile, sm, ex);
-  tile_done<SV, FAST>(P, tile, tc, ex);
+  tile_done<SV, FAST, LEARN == 0>(P, tile, tc, ex);
 }
 
 // ------------------------------------------------------------------------

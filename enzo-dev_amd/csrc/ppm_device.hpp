@@ -48,6 +48,33 @@ struct DevExec {
     f(tid, r);
     __syncthreads();
   }
+  // Phases of one pencil per wavefront (or several): the wavefront's LDS
+  // operations are in order, so only the compiler has to keep theirs.  The CPU
+  // execution runs work-items one by one: a barrier there.
+  static constexpr bool kWave = true;
+  __device__ static void wave_order() {
+#ifdef HIPCPU_RUNTIME
+    __syncthreads();
+#else
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#endif
+  }
+  template <class F>
+  __device__ void wave(F f) {
+    f(tid, r);
+    wave_order();
+  }
+  // what follows reads or writes LDS of other pencils (any), or has (spread)
+  __device__ void meet(bool any) {
+    if (any) __syncthreads();
+    else wave_order();
+  }
+  template <class F>
+  __device__ void spread(F f, bool any) {
+    f(tid, r);
+    meet(any);
+  }
   // a wavefront vote per wavefront, its population count in LDS, the sum
   // over the workgroup's wavefronts (at most 16: 1024 work-items)
   template <class F>
@@ -137,17 +164,25 @@ __device__ inline void flag_group(const SweepParams &P, int grp) {
 // fallback chain can cross segments) and settles them; with the HLL solver
 // there is no fallback and either is an error.
 // FAST: an operand out of range (Regs::oob) does the same.
-template <int SV, int FAST = 0>
+// WV: the tile's counts are per work-item (Regs), the wavefronts finish apart.
+template <int SV, int FAST = 0, bool WV = false>
 __device__ inline void tile_done(const SweepParams &P, int tile, const TileCounts &tc,
                                  const DevExec &ex) {
-  if constexpr (FAST != 0)
-    if (ex.r.oob) flag_group(P, tile / P.nseg);
-  if (threadIdx.x != 0) return;
-  if (tc.bad || tc.err) {
+  int bad, chains;
+  if constexpr (WV) {
+    bad = __ballot(ex.r.bad || (FAST != 0 && ex.r.oob)) != 0;
+    chains = __popcll(__ballot(ex.r.chains != 0));
+    if ((threadIdx.x & 63) != 0) return;
+  } else {
+    if (threadIdx.x != 0) return;
+    bad = tc.bad || tc.err;
+    chains = tc.chains;
+  }
+  if (bad) {
     if (SV == 0 || P.hllc) flag_group(P, tile / P.nseg);
     else atomicAdd(&P.counters[2], 1ull);
   }
-  if (tc.chains) atomicAdd(&P.counters[1], (unsigned long long)tc.chains);
+  if (chains) atomicAdd(&P.counters[1], (unsigned long long)chains);
 }
 
 // Every pencil of group `grp` (P.tp pencils along t1) redone whole with the

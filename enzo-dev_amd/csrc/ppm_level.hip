@@ -67,7 +67,7 @@ void level_sweep_kernel(const SweepParams *__restrict__ params, const Work *__re
   const Work w = work[xcd_tile((int)blockIdx.x, (int)gridDim.x)];
   const SweepParams &P = params[w.grid];
   const TileCounts tc = sweep_tile<TP, TS, UNI, DevExec, LEARN, SV, -1, FAST>(P, w.tile, sm, ex);
-  tile_done<SV, FAST>(P, w.tile, tc, ex);
+  tile_done<SV, FAST, LEARN == 0>(P, w.tile, tc, ex);
 }
 
 // The same sweep as one persistent launch: a few workgroups per CU, each
@@ -106,7 +106,7 @@ void level_sweep_persistent_kernel(const SweepParams *__restrict__ params,
     // and keeps them all live (spilling registers)
     PPM_OPAQUE_VGPR(ex.tid);
     const TileCounts tc = sweep_tile<TP, TS, UNI, DevExec, LEARN, 0, -1, FAST>(P, w.tile, sm, ex);
-    tile_done<0, FAST>(P, w.tile, tc, ex);
+    tile_done<0, FAST, LEARN == 0>(P, w.tile, tc, ex);
   }
   if (threadIdx.x == 0) {
     const unsigned nx = gridDim.x / nparts + ((int)(gridDim.x % nparts) > x ? 1u : 0u);
