@@ -72,7 +72,9 @@ inline bool uniform_axis(const double *dx, int N, const std::vector<double> &t, 
 // segments, 0 when none fits (or more than cap would be needed).
 template <int TP, int TS>
 inline int build_segments(int N, int i1, int i2, int *o, int *w, int cap) {
-  for (int nseg = (N + TS - 8) / (TS - 7); nseg <= N && nseg <= cap; nseg++) {
+  // (a segment inside the pencil owns at most TS - 7 cells, one at an end up
+  // to TS - 3, and a whole pencil of TS + 1 cells fits alone)
+  for (int nseg = (N + TS) / (TS + 1); nseg <= N && nseg <= cap; nseg++) {
     int base = N / nseg, rem = N % nseg, start = 1;
     bool ok = true;
     for (int s = 0; s < nseg; s++) {

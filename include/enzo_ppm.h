@@ -554,8 +554,9 @@ int hipPPMLevelUseGraph(hipPPMLevel *Level, enzo_int enable);
 int hipPPMLevelPersistent(hipPPMLevel *Level, enzo_int enable);
 
 /* Tile shape of grid `grid` along sweep axis `dim`: 0 = 16 pencils x 16
-   interfaces, 1 = 8 x 32 (default), 2 = 4 x 64; hipPPMLevelCommitShapes
-   rebuilds the work lists. */
+   interfaces, 1 = 8 x 32, 2 = 4 x 64 (the default is the shape with the
+   fewest lanes per pencil); hipPPMLevelCommitShapes rebuilds the work
+   lists. */
 int hipPPMLevelSetShape(hipPPMLevel *Level, enzo_int grid, enzo_int dim, enzo_int shape);
 int hipPPMLevelCommitShapes(hipPPMLevel *Level);
 

@@ -9,9 +9,10 @@ import oracle
 from enzo_ppm import abi, device, problems
 from helpers import DeviceArrays, cpu_library, field_report, noalloc_solve
 
-# owned cells per segment are at most 57 (4 x 64 tiles): 51 active cells fill
-# one segment with their ghosts, 52 need two, 108 / 109 two and three
-EDGES = [(51, 4, 5), (52, 5, 4), (4, 108, 3), (3, 4, 109), (2, 2, 3), (9, 12, 7)]
+# a pencil of 65 cells (59 active) is the longest in one segment of 4 x 64
+# tiles, of 122 (116) in two; 33 (27) in one of 8 x 32, 58 (52) in two
+EDGES = [(51, 4, 5), (52, 5, 4), (4, 108, 3), (3, 4, 109), (2, 2, 3), (9, 12, 7),
+         (59, 27, 2), (60, 28, 3), (2, 116, 53), (3, 117, 20)]
 
 
 def check(lib, active, solver, ncolours, dual, stretch=0.0, cycle=1):
@@ -195,3 +196,51 @@ def test_odd_states_gpu(kind):
         na, nb = np.isnan(a), np.isnan(b)
         assert np.array_equal(na, nb), kind
         assert np.array_equal(a[~na].view(np.uint64), b[~nb].view(np.uint64)), kind
+
+
+# Every tile shape of the batched level at the lengths where its segments
+# change: 16 x 16 holds 17 cells in one, 8 x 32 33, 4 x 64 65.
+LEVEL_ACTIVE = [(11, 12, 27), (28, 10, 11), (59, 11, 6), (60, 27, 7), (19, 53, 8)]
+
+
+def check_level_shapes(lib, solver):
+    from enzo_ppm.level import Level
+    grids = []
+    for k, a in enumerate(LEVEL_ACTIVE):
+        g, glob, run = problems.random_smooth(list(a), seed=k, ncolours=1)
+        g.fill_periodic()
+        for d in range(3):
+            g.cellwidth[d][...] = 1.0 / 64
+        grids.append(g)
+    glob["RiemannSolver"] = solver
+    dt = min(oracle.compute_time_step("port", g, glob, run["cfl"]) for g in grids)
+    refs = [g.copy() for g in grids]
+    for r in refs:
+        r.dt = dt
+        assert oracle.solve_ppm_de("port", r, glob, cycle=1)[0] == abi.SUCCESS
+    for shape in (None, 0, 1, 2):
+        work = [g.copy() for g in grids]
+        lv = Level(work, glob, lib=lib)
+        if shape is not None:
+            for k in range(len(work)):
+                for d in range(3):
+                    lv.set_shape(k, d, shape)
+            lv.commit_shapes()
+        lv.step(1, dt)
+        assert lv.status()[0] == abi.SUCCESS
+        lv.download()
+        lv.close()
+        for g, r in zip(work, refs):
+            for a, b in zip(g.fields, r.fields):
+                assert np.array_equal(a.view(np.uint64), b.view(np.uint64)), shape
+
+
+@ALL_SOLVERS
+def test_level_shapes_cpu(solver):
+    check_level_shapes(cpu_library(), solver)
+
+
+@pytest.mark.gpu
+@ALL_SOLVERS
+def test_level_shapes_gpu(solver):
+    check_level_shapes(None, solver)
