@@ -30,22 +30,21 @@ namespace {
 
 constexpr int kTP = kGridTP;  // pencils per workgroup
 constexpr int kTS = kGridTS;  // interfaces per pencil segment
-using SweepCfg = Cfg<kTP, kTS>;
 
 // ------------------------------------------------------------------------
 // Fused sweep kernel: see ppm_sweep.hpp for the stages.
 // DF 1: diffusion in one launch (wait_pair).  DF 0 keeps the tile's test of
 // P.idiff, never set there: it splits the Riemann phase, which the compiler
 // then schedules better (256^3 step 7.50 ms; 7.70 without the test).
-template <int UNI, int LEARN, int SV, int DF, int FAST>
+template <int UNI, int LEARN, int SV, int DF, int FAST, int TP = kTP, int TS = kTS>
 // 5 wavefronts per SIMD: 96 VGPRs (a few spilled) and 31 KB of LDS per
 // workgroup, 5 workgroups per CU.  The HLL / HLLC tile (SV) keeps more
 // interface values live: 4 wavefronts (116 VGPRs, 6 spilled) take 1.64 ms
 // per 160^3 HLLC step against 1.89 ms with 5 (24 spilled).  So do the fast
 // tiles (FAST; 110 VGPRs): 6.2 ms per 256^3 step, 6.65 with 5 (10 spilled).
-__global__ __launch_bounds__(kTP *kTS) __attribute__((amdgpu_waves_per_eu((SV == 0 && FAST == 0 ? 5 : 4))))
+__global__ __launch_bounds__(TP *TS) __attribute__((amdgpu_waves_per_eu((SV == 0 && FAST == 0 ? 5 : 4))))
 void ppm_sweep_kernel(SweepParams P) {
-  __shared__ double sm[SweepCfg::SMEM];
+  __shared__ double sm[Cfg<TP, TS>::SMEM];
   PPM_LDS_ENTER(sm);
   DevExec ex;
   int tile;
@@ -58,7 +57,7 @@ void ppm_sweep_kernel(SweepParams P) {
     tile = PPM_UNIFORM(turn);
   }
   const TileCounts tc =
-      sweep_tile<kTP, kTS, UNI, DevExec, LEARN, SV, DF == 0 ? -1 : DF, FAST>(P, tile, sm, ex);
+      sweep_tile<TP, TS, UNI, DevExec, LEARN, SV, DF == 0 ? -1 : DF, FAST>(P, tile, sm, ex);
   tile_done<SV, FAST, LEARN == 0>(P, tile, tc, ex);
 }
 
@@ -228,10 +227,10 @@ struct hipPPMData {
   int *fb_flag = nullptr;
   unsigned *fb_list = nullptr, *fb_state = nullptr;  // fb_state: count, done, diffusion's ticket
   long long fb_groups = 0;
-  int *segbuf = nullptr;  // per axis: o[nseg], w[nseg]
   int uni[3] = {0, 0, 0};  // axis has one cell width
   double kt[3][NTAB];      // its coefficient entries
-  int segoff[3] = {0, 0, 0}, nseg[3] = {0, 0, 0};
+  int nseg[3] = {0, 0, 0};            // segments of an axis in the 4 x 64 tiles
+  int shape[3] = {2, 2, 2}, nshape[3] = {0, 0, 0};  // its best shape and that one's segments
   // face capture
   int *face_head[3] = {nullptr, nullptr, nullptr};
   FaceRec *faces[3] = {nullptr, nullptr, nullptr};
@@ -344,7 +343,7 @@ void free_data(hipPPMData *D) {
   for (hipEvent_t e : D->ev) (void)hipEventDestroy(e);
   D->ev.clear();
   void *ptrs[] = {D->A, D->B, D->pres, D->xch, D->accel, D->tab[0], D->tab[1], D->tab[2], D->cwdev[0],
-                  D->cwdev[1], D->cwdev[2], D->flat, D->qc, D->dt, D->dtmin, D->counters, D->segbuf,
+                  D->cwdev[1], D->cwdev[2], D->flat, D->qc, D->dt, D->dtmin, D->counters,
                   D->fb_flag, D->fb_list, D->fb_state, D->learn, D->harvest, D->harvest_n,
                   D->cwdt[0], D->cwdt[1], D->cwdt[2], D->old,
                   D->face_head[0], D->face_head[1], D->face_head[2], D->faces[0], D->faces[1],
@@ -503,9 +502,6 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
   S.dim = dim; S.N = N; S.i1 = i1; S.i2 = i2; S.rank = rank;
   for (int d = 0; d < 3; d++) S.GD[d] = D->GD[d];
   S.cells = D->cells;
-  S.nseg = D->nseg[dim];
-  S.seg_o = D->segbuf + D->segoff[dim];
-  S.seg_w = D->segbuf + D->segoff[dim] + D->nseg[dim];
   S.A = D->A;
   S.B = D->B;
   S.ncol = (int)P->NumberOfColours;
@@ -550,7 +546,6 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
   S.fb_count = D->fb_state;
   S.fb_done = D->fb_state + 1;
   S.fb_tag = 0;
-  S.tp = kTP;
   S.fb_ok = pencil_fits<kFbTS>(S) ? 1 : 0;
   S.hllc = P->RiemannSolver == ENZO_PPM_RIEMANN_HLLC ? 1 : 0;
   S.learn = D->learned ? D->learn : nullptr;
@@ -565,9 +560,31 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
   const int variant = (S.uni[0] ? 1 : 0) | (D->learned ? 2 : 0);
   const bool two_shock = P->RiemannSolver == ENZO_PPM_RIEMANN_TWOSHOCK;
   const bool fast = set_fast(S) && two_shock && !D->learned && D->harvest_cap == 0;
+  // tile shape: the fast and the HLL / HLLC tiles of a uniform axis take the
+  // one with the fewest lanes per pencil (67-cell pencils: 3 x 32 instead of
+  // 2 x 64; 97x61x45 step 201 us instead of 211); the others 4 x 64
+  const int shape = S.uni[0] && S.idiff == 0 && (fast || !two_shock) ? D->shape[dim] : 2;
+  set_segments(S, shape == 2 ? D->nseg[dim] : D->nshape[dim]);
+  S.tp = kShapeTP[shape];
+  auto launch_shaped = [&](unsigned nblk, auto sv, auto fst) {
+    constexpr int SV = decltype(sv)::value, FST = decltype(fst)::value;
+    const dim3 g(nblk), b(256);
+    switch (shape) {
+      case 0: hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, SV, 0, FST, 16, 16>), g, b, 0, D->stream, S); break;
+      case 1: hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, SV, 0, FST, 8, 32>), g, b, 0, D->stream, S); break;
+      default: hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, SV, 0, FST>), g, b, 0, D->stream, S); break;
+    }
+    return hipGetLastError();
+  };
   auto launch_tiles = [&](unsigned nblk, auto diff) {
     constexpr int DF = decltype(diff)::value;
     const dim3 g(nblk), b(kTP * kTS);
+    if constexpr (DF == 0) {
+      using std::integral_constant;
+      if (!two_shock && S.uni[0])
+        return launch_shaped(nblk, integral_constant<int, 1>(), integral_constant<int, 0>());
+      if (fast) return launch_shaped(nblk, integral_constant<int, 0>(), integral_constant<int, 1>());
+    }
     if (!two_shock) {
       if (S.uni[0]) hipLaunchKernelGGL((ppm_sweep_kernel<1, 0, 1, DF, 0>), g, b, 0, D->stream, S);
       else hipLaunchKernelGGL((ppm_sweep_kernel<0, 0, 1, DF, 0>), g, b, 0, D->stream, S);
@@ -628,7 +645,7 @@ int launch_sweep(hipPPMData *D, const hipPPMParameter *P, double dtFixed, const 
   S.n_t2 = D->GD[S.ax_t2];
   S.t2_0 = 0;
   set_strides(S);
-  S.nblk_t1 = (S.n_t1 + kTP - 1) / kTP;
+  S.nblk_t1 = (S.n_t1 + S.tp - 1) / S.tp;
   const long long nblk = (long long)S.nseg * S.nblk_t1 * S.n_t2;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (D->profile && !S.pipe) {
@@ -681,25 +698,22 @@ int upload_geometry(hipPPMData *D, const hipPPMParameter *Para) {
   return ENZO_PPM_SUCCESS;
 }
 
-// Sweep segments of every axis into segs[] (o[nseg] then w[nseg] per axis,
-// D->segoff / D->nseg set); returns the number of ints or -1 when an axis
-// cannot be split.  segs holds 2 * 3 * ENZO_PPM_MAX_ANY_SINGLE_DIRECTION.
-int plan_segments(hipPPMData *D, const hipPPMParameter *Para, int *segs) {
-  int n = 0;
+// Sweep segments and best tile shape of every axis; false when an axis cannot
+// be split
+bool plan_segments(hipPPMData *D, const hipPPMParameter *Para) {
   for (int d = 0; d < 3; d++) {
     const int N = D->GD[d];
     const int i1 = (int)Para->GridStartIndex[d] + 1, i2 = (int)Para->GridEndIndex[d] + 1;
-    int ns = 0;
-    if (d < Para->GridRank && N > 1) {
-      ns = build_segments<kTP, kTS>(N, i1, i2, segs + n, segs + n + N, N);
-      if (ns == 0) return -1;
-      for (int k = 0; k < ns; k++) segs[n + ns + k] = segs[n + N + k];  // w after o
-    }
-    D->segoff[d] = n;
-    D->nseg[d] = ns;
-    n += 2 * ns;
+    D->nseg[d] = D->nshape[d] = 0;
+    if (d >= Para->GridRank || N <= 1) continue;
+    int n[kShapes];
+    shape_segments(N, i1, i2, n);
+    if (n[2] == 0) return false;
+    D->nseg[d] = n[2];
+    D->shape[d] = best_shape(n);
+    D->nshape[d] = n[D->shape[d]];
   }
-  return n;
+  return true;
 }
 
 // pencil groups of any sweep launch: ceil(n_t1 / kTP) * n_t2
@@ -873,15 +887,7 @@ int hipPPMInitData(hipPPMData **Data, const hipPPMParameter *Para, void *stream)
   // geometry tables and segments (cheap; rebuilt on every init)
   st = upload_geometry(D, Para);
   if (st != ENZO_PPM_SUCCESS) return st;
-  std::vector<int> segs(2 * 3 * (size_t)ENZO_PPM_MAX_ANY_SINGLE_DIRECTION);
-  const int nsegs = plan_segments(D, Para, segs.data());
-  if (nsegs < 0) return ENZO_PPM_ERR_ARGUMENT;
-  if (D->segbuf) (void)hipFree(D->segbuf);
-  D->segbuf = nullptr;
-  if (alloc_dev((void **)&D->segbuf, sizeof(int) * std::max(1, nsegs)))
-    return ENZO_PPM_ERR_HIP;
-  if (nsegs > 0)
-    HIPCHK(hipMemcpy(D->segbuf, segs.data(), sizeof(int) * nsegs, hipMemcpyHostToDevice));
+  if (!plan_segments(D, Para)) return ENZO_PPM_ERR_ARGUMENT;
   hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(64), 0, D->stream, D->counters, 4);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemsetAsync(D->fb_flag, 0, sizeof(int) * D->fb_groups, D->stream));
@@ -1203,10 +1209,7 @@ int hipPPMSolvePPM_DE_NoAlloc(const enzo_ppm_grid *g, const enzo_ppm_globals *gl
   D.fb_flag = sc.take<int>((size_t)D.fb_groups);
   D.fb_list = sc.take<unsigned>((size_t)D.fb_groups);
   D.fb_state = sc.take<unsigned>(3);
-  static thread_local int segs[2 * 3 * ENZO_PPM_MAX_ANY_SINGLE_DIRECTION];
-  const int nsegs = plan_segments(&D, &Para, segs);
-  if (nsegs < 0) return ENZO_PPM_ERR_ARGUMENT;
-  D.segbuf = sc.take<int>((size_t)std::max(1, nsegs));
+  if (!plan_segments(&D, &Para)) return ENZO_PPM_ERR_ARGUMENT;
   if (Para.PPMDiffusionParameter != 0 && sc.used + 256 + sizeof(double) * cells <= kScratchBytes)
     D.xch = sc.take<double>(cells);  // else the exchange stays in the state's own arrays
   if (sc.used > kScratchBytes) {
@@ -1234,10 +1237,6 @@ int hipPPMSolvePPM_DE_NoAlloc(const enzo_ppm_grid *g, const enzo_ppm_globals *gl
   HIPCHK(hipGetLastError());
   st = upload_geometry(&D, &Para);
   if (st != ENZO_PPM_SUCCESS) return st;
-  if (nsegs > 0) {
-    HIPCHK(hipMemcpyAsync(D.segbuf, segs, sizeof(int) * nsegs, hipMemcpyHostToDevice, D.stream));
-    HIPCHK(hipStreamSynchronize(D.stream));  // segs is reused by the next call of this thread
-  }
   hipLaunchKernelGGL(gather_slots_kernel, dim3(grid_blocks((long long)cells * D.nslot)), dim3(256),
                      0, D.stream, D.A, D.cells, D.nslot, F);
   HIPCHK(hipGetLastError());

@@ -94,6 +94,30 @@ inline int build_segments(int N, int i1, int i2, int *o, int *w, int cap) {
   }
   return 0;
 }
+// the number of segments alone (0: none fits)
+template <int TP, int TS>
+inline int count_segments(int N, int i1, int i2) {
+  static thread_local int o[ENZO_PPM_MAX_ANY_SINGLE_DIRECTION], w[ENZO_PPM_MAX_ANY_SINGLE_DIRECTION];
+  return build_segments<TP, TS>(N, i1, i2, o, w,
+                                N < ENZO_PPM_MAX_ANY_SINGLE_DIRECTION ? N : ENZO_PPM_MAX_ANY_SINGLE_DIRECTION);
+}
+// Tile shapes of 256 work-items, pencils x interfaces; segments of each that
+// an axis takes, and the one with the fewest lanes per pencil (of equals the
+// longest segments: the fewest halo loads).
+constexpr int kShapes = 3;
+constexpr int kShapeTP[kShapes] = {16, 8, 4};
+constexpr int kShapeTS[kShapes] = {16, 32, 64};
+inline void shape_segments(int N, int i1, int i2, int n[kShapes]) {
+  n[0] = count_segments<16, 16>(N, i1, i2);
+  n[1] = count_segments<8, 32>(N, i1, i2);
+  n[2] = count_segments<4, 64>(N, i1, i2);
+}
+inline int best_shape(const int n[kShapes]) {
+  int best = -1;
+  for (int s = 0; s < kShapes; s++)
+    if (n[s] > 0 && (best < 0 || n[s] * kShapeTS[s] <= n[best] * kShapeTS[best])) best = s;
+  return best;
+}
 template <int TP, int TS>
 inline bool build_segments(int N, int i1, int i2, std::vector<int> &o, std::vector<int> &w) {
   o.assign(N, 0);

@@ -53,11 +53,6 @@ struct GridGeom {
   int GD[3];
 };
 
-// tile shapes of the level kernels (256 work-items each)
-constexpr int kShapes = 3;
-constexpr int kShapeTP[kShapes] = {16, 8, 4};
-constexpr int kShapeTS[kShapes] = {16, 32, 64};
-
 template <int TP, int TS, int UNI, int LEARN, int SV, int FAST>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((SV == 0 && FAST == 0 ? 5 : 4))))
 void level_sweep_kernel(const SweepParams *__restrict__ params, const Work *__restrict__ work) {
@@ -271,17 +266,6 @@ bool dev_alloc(T **p, size_t n) {
   return hipMalloc((void **)p, sizeof(T) * std::max<size_t>(n, 1)) != hipSuccess;
 }
 
-template <int TP, int TS>
-bool segments_for(int N, int i1, int i2, std::vector<int> &o, std::vector<int> &w) {
-  return build_segments<TP, TS>(N, i1, i2, o, w);
-}
-
-bool segments_shape(int s, int N, int i1, int i2, std::vector<int> &o, std::vector<int> &w) {
-  if (s == 0) return segments_for<16, 16>(N, i1, i2, o, w);
-  if (s == 1) return segments_for<8, 32>(N, i1, i2, o, w);
-  return segments_for<4, 64>(N, i1, i2, o, w);
-}
-
 }  // namespace
 
 struct hipPPMLevel {
@@ -297,16 +281,12 @@ struct hipPPMLevel {
   std::vector<int> uni;             // 3 per grid
   std::vector<double> kt;           // 3 * NTAB per grid
   std::vector<int> shape;           // 3 per grid: tile shape index per sweep axis
-  // segments per (grid, axis, shape): o then w, in segs
-  std::vector<int> hsegs;
-  std::vector<long long> seg_off;   // ((g * 3 + d) * kShapes + s) -> offset into segs
-  std::vector<int> seg_n;
+  std::vector<int> seg_n;           // segments per (grid, axis, shape)
   std::vector<long long> grp_off;   // fallback group flags per grid
   long long ngroups = 0;
   // device memory
   double *A = nullptr, *B = nullptr, *pres = nullptr, *accel = nullptr;
   double *tabs = nullptr, *cws = nullptr, *flat = nullptr, *qc = nullptr;
-  int *segs = nullptr;
   double *dt = nullptr;
   unsigned long long *dtmin = nullptr, *counters = nullptr;
   int *fb_flag = nullptr;
@@ -415,7 +395,7 @@ void face_params(const hipPPMLevel *L, int g, int d, SweepParams &S) {
 void free_level(hipPPMLevel *L) {
   drop_graphs(L);
   for (auto &F : L->faces) free_faces(F);
-  void *ptrs[] = {L->A, L->B, L->pres, L->accel, L->tabs, L->cws, L->flat, L->qc, L->segs, L->dt,
+  void *ptrs[] = {L->A, L->B, L->pres, L->accel, L->tabs, L->cws, L->flat, L->qc, L->dt,
                   L->dtmin, L->counters, L->fb_flag, L->fb_list, L->fb_state, L->grp_grid,
                   L->dgrp_off, L->dparams,
                   L->dflat, L->dpres, L->dwork, L->dpwork, L->learn, L->cws_dt, L->old,
@@ -583,10 +563,7 @@ int build_plan(hipPPMLevel *L) {
         set_strides(S);
         S.tp = kShapeTP[s];
         S.nblk_t1 = (S.n_t1 + S.tp - 1) / S.tp;
-        const long long so = L->seg_off[((size_t)g * 3 + d) * kShapes + s];
-        S.nseg = L->seg_n[((size_t)g * 3 + d) * kShapes + s];
-        S.seg_o = L->segs + so;
-        S.seg_w = L->segs + so + S.nseg;
+        set_segments(S, L->seg_n[((size_t)g * 3 + d) * kShapes + s]);
         double *src = par == 0 ? L->A : L->B, *dst = par == 0 ? L->B : L->A;
         S.A = src + L->off[g];
         S.B = dst + L->off[g];
@@ -878,7 +855,6 @@ int hipPPMLevelCreate(hipPPMLevel **Level, enzo_int NumberOfGrids, const hipPPMP
   L->uni.resize(3 * G);
   L->kt.assign((size_t)3 * G * NTAB, 0.0);
   L->shape.assign(3 * G, 1);
-  L->seg_off.assign((size_t)G * 3 * kShapes, 0);
   L->seg_n.assign((size_t)G * 3 * kShapes, 0);
   long long tot = 0, ptot = 0, ttot = 0, wtot = 0, ftot = 0, qtot = 0;
   for (int g = 0; g < G; g++) {
@@ -917,30 +893,15 @@ int hipPPMLevelCreate(hipPPMLevel **Level, enzo_int NumberOfGrids, const hipPPMP
     for (int d = 0; d < L->rank; d++) {
       const int N = L->GD[3 * g + d];
       const int i1 = (int)Para[g].GridStartIndex[d] + 1, i2 = (int)Para[g].GridEndIndex[d] + 1;
-      for (int s = 0; s < kShapes; s++) {
-        std::vector<int> o, w;
-        const size_t k = ((size_t)g * 3 + d) * kShapes + s;
-        L->seg_off[k] = (long long)L->hsegs.size();
-        if (!segments_shape(s, N, i1, i2, o, w)) continue;
-        L->seg_n[k] = (int)o.size();
-        L->hsegs.insert(L->hsegs.end(), o.begin(), o.end());
-        L->hsegs.insert(L->hsegs.end(), w.begin(), w.end());
-      }
-      const int *n = &L->seg_n[((size_t)g * 3 + d) * kShapes];
+      int *n = &L->seg_n[((size_t)g * 3 + d) * kShapes];
+      shape_segments(N, i1, i2, n);
       if (n[1] == 0) {
         delete L;
         return ENZO_PPM_ERR_ARGUMENT;
       }
-      // the default shape: the fewest lanes per pencil, segments times
-      // interfaces (of equals the longest segments: the fewest halo loads).
-      // 512 grids of 8..64 cells an axis: 5.7 ms per level step, 6.4 with
-      // 8 x 32 everywhere, 7.9 with 4 x 64.
-      int best = 1;
-      for (int s = 0; s < kShapes; s++)
-        if (n[s] > 0 && n[s] * kShapeTS[s] <= n[best] * kShapeTS[best] &&
-            (n[s] * kShapeTS[s] < n[best] * kShapeTS[best] || kShapeTS[s] > kShapeTS[best]))
-          best = s;
-      L->shape[3 * g + d] = best;
+      // the default shape: 512 grids of 8..64 cells an axis take 5.7 ms per
+      // level step, 6.4 with 8 x 32 everywhere, 7.9 with 4 x 64
+      L->shape[3 * g + d] = best_shape(n);
     }
   long long ngroups = 0;
   std::vector<int> hgrp_grid;
@@ -973,7 +934,7 @@ int hipPPMLevelCreate(hipPPMLevel **Level, enzo_int NumberOfGrids, const hipPPMP
   if (dev_alloc(&L->A, tot) || dev_alloc(&L->B, tot) || dev_alloc(&L->pres, ptot) ||
       (L->gravity && dev_alloc(&L->accel, 3 * ptot)) || dev_alloc(&L->tabs, ttot) ||
       dev_alloc(&L->cws, wtot) || dev_alloc(&L->flat, ftot) || dev_alloc(&L->qc, qtot) ||
-      dev_alloc(&L->segs, L->hsegs.size()) || dev_alloc(&L->dt, 1) || dev_alloc(&L->dtmin, 1) ||
+      dev_alloc(&L->dt, 1) || dev_alloc(&L->dtmin, 1) ||
       dev_alloc(&L->counters, 4) || dev_alloc(&L->fb_flag, ngroups) ||
       dev_alloc(&L->fb_list, ngroups) || dev_alloc(&L->fb_state, 2) ||
       dev_alloc(&L->grp_grid, ngroups) || dev_alloc(&L->dgrp_off, G) ||
@@ -993,9 +954,7 @@ int hipPPMLevelCreate(hipPPMLevel **Level, enzo_int NumberOfGrids, const hipPPMP
       L->persistent_blocks = 4 * ncu;
   }
   if (upload_geometry(L) != ENZO_PPM_SUCCESS) return fail(ENZO_PPM_ERR_HIP);
-  if ((!L->hsegs.empty() && hipMemcpy(L->segs, L->hsegs.data(), sizeof(int) * L->hsegs.size(),
-                                      hipMemcpyHostToDevice) != hipSuccess) ||
-      hipMemcpy(L->dpwork, pw.data(), sizeof(Work) * pw.size(), hipMemcpyHostToDevice) != hipSuccess ||
+  if (hipMemcpy(L->dpwork, pw.data(), sizeof(Work) * pw.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(L->fb_flag, 0, sizeof(int) * ngroups) != hipSuccess ||
       hipMemcpy(L->grp_grid, hgrp_grid.data(), sizeof(int) * ngroups, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(L->dgrp_off, hgrp_off.data(), sizeof(unsigned) * G, hipMemcpyHostToDevice) != hipSuccess ||

@@ -217,7 +217,10 @@ struct SweepParams {
   int st_s, st_1, st_2;   // grid strides of the sweep, t1 and t2 axes (set_strides)
   int n_t1, n_t2, t2_0;   // pencil counts; first t2 (slab-serial launches)
   int nseg, nblk_t1;
-  const int *seg_o, *seg_w;  // owned cells of each segment: [o, o+w)
+  // owned cells of each segment: N / nseg, one more in the first N % nseg
+  // (set_segments), or [o, o+w) from tables
+  int seg_base, seg_rem;
+  const int *seg_o, *seg_w;
   const double *A;        // source state  (slot*cells + index)
   double *B;              // destination state
   int ncol;
@@ -558,6 +561,14 @@ PPM_HD int xcd_tile(int b, int nblk) {
   return x * q + (x < rem ? x : rem) + k;
 }
 
+// nseg segments as build_segments splits them
+inline void set_segments(SweepParams &S, int nseg) {
+  S.nseg = nseg;
+  S.seg_base = nseg > 0 ? S.N / nseg : 0;
+  S.seg_rem = nseg > 0 ? S.N % nseg : 0;
+  S.seg_o = S.seg_w = nullptr;
+}
+
 // interface and load ranges of a tile that owns cells [T.o, T.o + T.w)
 PPM_HD void tile_ranges(const SweepParams &P, Tile &T) {
   T.IA = T.o - 1 > P.i1 ? T.o - 1 : P.i1;
@@ -580,8 +591,13 @@ PPM_HD Tile make_tile(const SweepParams &P, int block) {
   T.t2 = P.t2_0 + r / P.nblk_t1;
   T.t1_0 = tb * TP;
   T.np = P.n_t1 - T.t1_0 < TP ? P.n_t1 - T.t1_0 : TP;
-  T.o = as_global(P.seg_o)[seg];
-  T.w = as_global(P.seg_w)[seg];
+  if (P.seg_o) {
+    T.o = as_global(P.seg_o)[seg];
+    T.w = as_global(P.seg_w)[seg];
+  } else {
+    T.o = 1 + seg * P.seg_base + (seg < P.seg_rem ? seg : P.seg_rem);
+    T.w = P.seg_base + (seg < P.seg_rem ? 1 : 0);
+  }
   tile_ranges(P, T);
   T.dt = dtval(P);
   T.qcu = qc_uniform(P, T.dt);
