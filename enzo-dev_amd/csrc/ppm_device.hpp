@@ -329,55 +329,70 @@ __device__ inline void block_min_dt(double local, unsigned long long *dtmin) {
 }
 
 // ------------------------------------------------------------------------
-// Periodic ghost fill along one axis (the periodic case of
-// ExternalBoundary::SetExternalBoundary): item gid copies one ghost cell of
-// one slot from the opposite side of the active region.
+// Periodic ghost fill (the periodic case of
+// ExternalBoundary::SetExternalBoundary) of every axis at once: filling x,
+// then y, then z gives every ghost cell the active cell its coordinates wrap
+// to, so each takes that one directly; only active cells are read and only
+// ghost cells written, and one launch does what one per axis did.
 struct BCParams {
-  int axis, ghost, nslot;
-  int GD[3], act[3];
+  int nslot;
+  int GD[3], act[3], ghost[3];  // ghost 0 on axes that are not filled
   long long cells;
   double *S;
 };
 
-// Whether the periodic fill of B's axis is defined and fits its items:
-// as many ghost cells on the right (`right_ghost`) as on the left, an
-// active extent of at least the ghost count (each ghost cell is then one
-// period from an active cell, the images CopyZonesFromGrid takes; a
-// narrower grid would also read ghost cells the same launch writes), and
-// fewer than 2^31 items.
-inline bool periodic_fits(const BCParams &B, long long right_ghost) {
-  const int a = B.axis;
-  const long long n = 2LL * B.ghost * B.GD[(a + 1) % 3] * B.GD[(a + 2) % 3] * B.nslot;
-  return right_ghost == B.ghost && B.ghost >= 0 && B.act[a] >= B.ghost && n < (1LL << 31);
+// Whether the fill of axis a is defined and fits its items: as many ghost
+// cells on the right (`right_ghost`) as on the left, an active extent of at
+// least the ghost count (each ghost cell is then one period from an active
+// cell, the images CopyZonesFromGrid takes), and fewer than 2^31 items.
+inline bool periodic_fits(const BCParams &B, int a, long long right_ghost) {
+  const long long n = 2LL * B.ghost[a] * B.GD[(a + 1) % 3] * B.GD[(a + 2) % 3] * B.nslot;
+  return right_ghost == B.ghost[a] && B.ghost[a] >= 0 && B.act[a] >= B.ghost[a] && n < (1LL << 31);
 }
 
-__device__ inline long long periodic_items(const BCParams &B) {
-  return (long long)2 * B.ghost * B.GD[(B.axis + 1) % 3] * B.GD[(B.axis + 2) % 3] * B.nslot;
+// ghost cells of the filled axes: z layers over the whole plane, y layers of
+// the active z, x layers of the active rows
+PPM_HD int periodic_cells(const BCParams &B, int n[3]) {
+  n[2] = 2 * B.ghost[2] * B.GD[1] * B.GD[0];
+  n[1] = B.act[2] * 2 * B.ghost[1] * B.GD[0];
+  n[0] = B.act[2] * B.act[1] * 2 * B.ghost[0];
+  return n[0] + n[1] + n[2];
 }
 
-// Item gid walks the box of the axis' ghost layers (extent 2 * ghost along
-// the axis, the grid's extent across it) with x fastest, so that the loads
-// and stores of a wavefront are contiguous along x (runs of `ghost` cells
-// when the axis is x).  Layer l < ghost is left ghost cell l, taken from
-// active cell l + act; layer l >= ghost is right ghost cell l + act, taken
-// from active cell l (act >= ghost, checked on the host).  The host also
-// keeps the item count below 2^31, so 32-bit arithmetic.
-__device__ inline void periodic_item(const BCParams &B, int gid) {
-  const int a = B.axis, g = B.ghost, act = B.act[a];
-  const int n0 = a == 0 ? 2 * g : B.GD[0], n1 = a == 1 ? 2 * g : B.GD[1],
-            n2 = a == 2 ? 2 * g : B.GD[2];
-  const int per_slot = n0 * n1 * n2;
-  const int slot = gid / per_slot;
-  int r = gid - slot * per_slot;
-  const int x0 = r % n0;
-  r /= n0;
-  const int x1 = r % n1, x2 = r / n1;
-  const int l = a == 0 ? x0 : a == 1 ? x1 : x2;
-  const int sa = a == 0 ? 1 : a == 1 ? B.GD[0] : B.GD[0] * B.GD[1];  // stride of the axis
-  const int base = (x2 * B.GD[1] + x1) * B.GD[0] + x0 - l * sa;     // cell 0 of the line
-  const int dst = l < g ? l : l + act, src = l < g ? l + act : l;
-  double *S = B.S + (long long)slot * B.cells;
-  S[base + dst * sa] = S[base + src * sa];
+// Ghost cell q, every slot (their loads in flight together); x fastest, so that
+// a wavefront's accesses are contiguous along x (runs of `ghost` cells in the
+// x layers).
+__device__ inline void periodic_cell(const BCParams &B, int q) {
+  int n[3];
+  periodic_cells(B, n);
+  int x[3];
+  if (q < n[2]) {
+    x[0] = q % B.GD[0];
+    q /= B.GD[0];
+    x[1] = q % B.GD[1];
+    x[2] = q / B.GD[1];
+    if (x[2] >= B.ghost[2]) x[2] += B.act[2];
+  } else if (q < n[2] + n[1]) {
+    q -= n[2];
+    x[0] = q % B.GD[0];
+    q /= B.GD[0];
+    x[1] = q % (2 * B.ghost[1]);
+    x[2] = B.ghost[2] + q / (2 * B.ghost[1]);
+    if (x[1] >= B.ghost[1]) x[1] += B.act[1];
+  } else {
+    q -= n[2] + n[1];
+    x[0] = q % (2 * B.ghost[0]);
+    q /= 2 * B.ghost[0];
+    x[1] = B.ghost[1] + q % B.act[1];
+    x[2] = B.ghost[2] + q / B.act[1];
+    if (x[0] >= B.ghost[0]) x[0] += B.act[0];
+  }
+  int y[3];
+  for (int a = 0; a < 3; a++)
+    y[a] = x[a] < B.ghost[a] ? x[a] + B.act[a] : x[a] >= B.ghost[a] + B.act[a] ? x[a] - B.act[a] : x[a];
+  double *D = B.S + ((long long)(x[2] * B.GD[1] + x[1]) * B.GD[0] + x[0]);
+  const double *F = B.S + ((long long)(y[2] * B.GD[1] + y[1]) * B.GD[0] + y[0]);
+  for (int s = 0; s < B.nslot; s++) D[s * B.cells] = F[s * B.cells];
 }
 
 // ------------------------------------------------------------------------

@@ -215,12 +215,13 @@ __global__ __launch_bounds__(64) void level_copy_kernel(const CopyBox *__restric
   }
 }
 
-// periodic ghost fill of every grid along one axis: one workgroup row per grid
-__global__ void level_periodic_kernel(const BCParams *__restrict__ B) {
+// periodic ghost fill of every grid: one workgroup row per grid
+__global__ __launch_bounds__(256) void level_periodic_kernel(const BCParams *__restrict__ B) {
   const BCParams &b = B[blockIdx.y];
-  const int n = (int)periodic_items(b);  // below 2^31 (periodic_fits)
-  for (int gid = blockIdx.x * blockDim.x + threadIdx.x; gid < n; gid += gridDim.x * blockDim.x)
-    periodic_item(b, gid);
+  int n[3];
+  const int cells = periodic_cells(b, n);
+  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < cells; q += gridDim.x * blockDim.x)
+    periodic_cell(b, q);
 }
 
 // one domain face of every grid in the list (blockIdx.y)
@@ -1459,35 +1460,33 @@ int hipPPMLevelPeriodicBoundary(hipPPMLevel *L) {
   if (!L) return ENZO_PPM_ERR_ARGUMENT;
   L->pres_current = false;  // the state changes
   const int G = L->ngrids;
-  std::vector<BCParams> hb((size_t)3 * G);
-  long long nmax = 1;
-  for (int a = 0; a < L->rank; a++)
-    for (int g = 0; g < G; g++) {
-      const hipPPMParameter &P = L->para[g];
-      BCParams &B = hb[(size_t)a * G + g];
-      B.axis = a;
-      B.ghost = (int)P.GridStartIndex[a];
-      B.nslot = L->nslot;
-      for (int d = 0; d < 3; d++) {
-        B.GD[d] = L->GD[3 * g + d];
-        B.act[d] = (int)(P.GridEndIndex[d] - P.GridStartIndex[d] + 1);
-      }
-      if (!periodic_fits(B, P.GridDimension[a] - P.GridEndIndex[a] - 1)) return ENZO_PPM_ERR_ARGUMENT;
-      B.cells = L->cells[g];
-      B.S = (L->parity == 0 ? L->A : L->B) + L->off[g];
-      nmax = std::max(nmax, (long long)2 * B.ghost * B.GD[(a + 1) % 3] * B.GD[(a + 2) % 3] *
-                                B.nslot);
+  std::vector<BCParams> hb(G);
+  int nmax = 1;
+  for (int g = 0; g < G; g++) {
+    const hipPPMParameter &P = L->para[g];
+    BCParams &B = hb[g];
+    B.nslot = L->nslot;
+    B.cells = L->cells[g];
+    B.S = (L->parity == 0 ? L->A : L->B) + L->off[g];
+    for (int d = 0; d < 3; d++) {
+      B.GD[d] = L->GD[3 * g + d];
+      B.act[d] = d < L->rank ? (int)(P.GridEndIndex[d] - P.GridStartIndex[d] + 1) : B.GD[d];
+      B.ghost[d] = d < L->rank ? (int)P.GridStartIndex[d] : 0;
     }
+    for (int a = 0; a < L->rank; a++)
+      if (!periodic_fits(B, a, P.GridDimension[a] - P.GridEndIndex[a] - 1)) return ENZO_PPM_ERR_ARGUMENT;
+    int n[3];
+    nmax = std::max(nmax, periodic_cells(B, n));
+  }
   BCParams *db = nullptr;
   if (dev_alloc(&db, hb.size())) return ENZO_PPM_ERR_HIP;
   int st = ENZO_PPM_SUCCESS;
   if (hipMemcpyAsync(db, hb.data(), sizeof(BCParams) * hb.size(), hipMemcpyHostToDevice,
                      L->stream) != hipSuccess)
     st = ENZO_PPM_ERR_HIP;
-  const unsigned bx = (unsigned)std::min<long long>((nmax + 255) / 256, 65535);
-  for (int a = 0; a < L->rank && st == ENZO_PPM_SUCCESS; a++) {
-    hipLaunchKernelGGL(level_periodic_kernel, dim3(bx, (unsigned)G), dim3(256), 0, L->stream,
-                       db + (size_t)a * G);
+  const unsigned bx = (unsigned)((nmax + 255) / 256);
+  if (st == ENZO_PPM_SUCCESS) {
+    hipLaunchKernelGGL(level_periodic_kernel, dim3(bx, (unsigned)G), dim3(256), 0, L->stream, db);
     if (hipGetLastError() != hipSuccess) st = ENZO_PPM_ERR_HIP;
   }
   if (hipStreamSynchronize(L->stream) != hipSuccess) st = ENZO_PPM_ERR_HIP;
