@@ -234,12 +234,18 @@ struct hipPPMData {
   long long fb_groups = 0;
   int uni[3] = {0, 0, 0};  // axis has one cell width
   double kt[3][NTAB];      // its coefficient entries
+  // host copies of the sweep widths on the device (upload_geometry), and
+  // whether an axis' tables there are theirs
+  bool keep_geometry = false;
+  std::vector<double> hdx[3];
+  bool geometry[3] = {false, false, false};
   int nseg[3] = {0, 0, 0};            // segments of an axis in the 4 x 64 tiles
   int shape[3] = {2, 2, 2}, nshape[3] = {0, 0, 0};  // its best shape and that one's segments
   // face capture
   int *face_head[3] = {nullptr, nullptr, nullptr};
   FaceRec *faces[3] = {nullptr, nullptr, nullptr};
   double *face_out[3] = {nullptr, nullptr, nullptr};
+  size_t head_cap[3] = {0, 0, 0}, rec_cap[3] = {0, 0, 0}, out_cap[3] = {0, 0, 0};  // elements held
   std::vector<FaceRec> hfaces[3];
   std::vector<int> hface_sub[3], hface_side[3];
   long long face_total[3] = {0, 0, 0};
@@ -267,13 +273,7 @@ struct hipPPMData {
   int profile = 0;
   std::vector<hipEvent_t> ev;  // pairs
   size_t ev_used = 0;
-  // pinned staging ring of the host-array transfers (stage_upload /
-  // stage_download), allocated on first use; stage_busy[b]: a copy into or
-  // out of buffer b was queued and stage_ev[b] marks its end
-  void *stage[3] = {nullptr, nullptr, nullptr};
-  hipEvent_t stage_ev[3] = {nullptr, nullptr, nullptr};
-  bool stage_busy[3] = {false, false, false};
-  int stage_next = 0;
+  StageRing ring;  // pinned staging of the host-array transfers, on first use
 };
 
 namespace {
@@ -343,6 +343,18 @@ bool alloc_dev(void **p, size_t bytes) {
   return false;
 }
 
+// *p to hold n elements at least (the contents are not kept); true when that
+// failed
+template <class T>
+bool grow_dev(T **p, size_t &cap, size_t n) {
+  if (*p && cap >= n) return false;
+  if (*p) (void)hipFree(*p);
+  cap = 0;
+  if (alloc_dev((void **)p, sizeof(T) * n)) return true;
+  cap = n;
+  return false;
+}
+
 void free_data(hipPPMData *D) {
   if (!D) return;
   for (hipEvent_t e : D->ev) (void)hipEventDestroy(e);
@@ -355,117 +367,36 @@ void free_data(hipPPMData *D) {
                   D->faces[2], D->face_out[0], D->face_out[1], D->face_out[2]};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
-  for (int b = 0; b < 3; b++) {
-    if (D->stage_ev[b]) (void)hipEventDestroy(D->stage_ev[b]);
-    if (D->stage[b]) (void)hipHostFree(D->stage[b]);
-    D->stage_ev[b] = nullptr;
-    D->stage[b] = nullptr;
-  }
+  D->ring.release();
 }
 
 // ------------------------------------------------------------------------
-// Host-array transfers.  hipMemcpy from the caller's pageable arrays moves
-// ~28 GB/s to the device and ~18 GB/s back (the runtime stages them
-// itself); here a field goes in chunks through a ring of pinned buffers,
-// the host copy of each chunk (CopyPool, several threads) overlapping the
-// DMA of the previous one, which runs at ~57 GB/s.  Smaller transfers, or a
-// host that cannot pin the ring, take the direct path.
-constexpr int kStageBufs = 3;
-constexpr size_t kStageBytes = size_t(32) << 20;  // per pinned buffer
-constexpr size_t kStageMin = size_t(8) << 20;     // direct path below this total
-
-struct HostXfer {
-  char *dst;
-  const char *src;
-  size_t bytes;
-};
-
-bool stage_ready(hipPPMData *D) {
-  if (D->stage[kStageBufs - 1]) return true;
-  for (int b = 0; b < kStageBufs; b++) {
-    if (!D->stage[b] && hipHostMalloc(&D->stage[b], kStageBytes, hipHostMallocDefault) != hipSuccess) {
-      D->stage[b] = nullptr;
-      return false;
-    }
-    if (!D->stage_ev[b] && hipEventCreateWithFlags(&D->stage_ev[b], hipEventDisableTiming) != hipSuccess) {
-      D->stage_ev[b] = nullptr;
-      (void)hipHostFree(D->stage[b]);
-      D->stage[b] = nullptr;
-      return false;
-    }
-  }
-  return true;
-}
-
-size_t xfer_total(const std::vector<HostXfer> &xs) {
-  size_t t = 0;
-  for (const HostXfer &x : xs) t += x.bytes;
-  return t;
-}
+// Host-array transfers through the handle's ring of pinned buffers; small
+// ones, or with a host that cannot pin it, directly.
+constexpr size_t kStageMin = size_t(8) << 20;
 
 // host -> device on D->stream; the caller's arrays may be reused on return
-// (the DMA reads only the pinned ring)
 int stage_upload(hipPPMData *D, const std::vector<HostXfer> &xs) {
-  if (xfer_total(xs) < kStageMin || !stage_ready(D)) {
+  const size_t n = StageRing::total(xs);
+  if (n < kStageMin || !D->ring.reserve(n)) {
     for (const HostXfer &x : xs)
       HIPCHK(hipMemcpyAsync(x.dst, x.src, x.bytes, hipMemcpyHostToDevice, D->stream));
     return ENZO_PPM_SUCCESS;
   }
-  int b = D->stage_next;
-  for (const HostXfer &x : xs)
-    for (size_t off = 0; off < x.bytes; off += kStageBytes) {
-      const size_t len = std::min(kStageBytes, x.bytes - off);
-      if (D->stage_busy[b]) HIPCHK(hipEventSynchronize(D->stage_ev[b]));
-      CopyPool::get().copy(D->stage[b], x.src + off, len);
-      HIPCHK(hipMemcpyAsync(x.dst + off, D->stage[b], len, hipMemcpyHostToDevice, D->stream));
-      HIPCHK(hipEventRecord(D->stage_ev[b], D->stream));
-      D->stage_busy[b] = true;
-      b = (b + 1) % kStageBufs;
-    }
-  D->stage_next = b;
+  HIPCHK(D->ring.upload(D->stream, xs));
   return ENZO_PPM_SUCCESS;
 }
 
 // device -> host after the work queued on D->stream; complete on return
 int stage_download(hipPPMData *D, const std::vector<HostXfer> &xs) {
-  if (xfer_total(xs) < kStageMin || !stage_ready(D)) {
+  const size_t n = StageRing::total(xs);
+  if (n < kStageMin || !D->ring.reserve(n)) {
     for (const HostXfer &x : xs)
       HIPCHK(hipMemcpyAsync(x.dst, x.src, x.bytes, hipMemcpyDeviceToHost, D->stream));
     HIPCHK(hipStreamSynchronize(D->stream));
     return ENZO_PPM_SUCCESS;
   }
-  char *pend_dst[kStageBufs] = {};
-  size_t pend_len[kStageBufs] = {};
-  auto drain = [&](int c) -> int {  // buffer c's chunk to the caller's array
-    if (!pend_dst[c]) return ENZO_PPM_SUCCESS;
-    HIPCHK(hipEventSynchronize(D->stage_ev[c]));
-    CopyPool::get().copy(pend_dst[c], D->stage[c], pend_len[c]);
-    pend_dst[c] = nullptr;
-    D->stage_busy[c] = false;
-    return ENZO_PPM_SUCCESS;
-  };
-  int b = D->stage_next;
-  for (const HostXfer &x : xs)
-    for (size_t off = 0; off < x.bytes; off += kStageBytes) {
-      const size_t len = std::min(kStageBytes, x.bytes - off);
-      if (pend_dst[b]) {
-        const int st = drain(b);
-        if (st != ENZO_PPM_SUCCESS) return st;
-      } else if (D->stage_busy[b]) {
-        HIPCHK(hipEventSynchronize(D->stage_ev[b]));
-      }
-      HIPCHK(hipMemcpyAsync(D->stage[b], x.src + off, len, hipMemcpyDeviceToHost, D->stream));
-      HIPCHK(hipEventRecord(D->stage_ev[b], D->stream));
-      D->stage_busy[b] = true;
-      pend_dst[b] = x.dst + off;
-      pend_len[b] = len;
-      b = (b + 1) % kStageBufs;
-    }
-  for (int i = 0; i < kStageBufs; i++) {
-    const int st = drain((b + i) % kStageBufs);
-    if (st != ENZO_PPM_SUCCESS) return st;
-  }
-  D->stage_next = b;
+  HIPCHK(D->ring.download(D->stream, xs));
   return ENZO_PPM_SUCCESS;
 }
 
@@ -685,10 +616,17 @@ int upload_geometry(hipPPMData *D, const hipPPMParameter *Para) {
   static thread_local double cw[kN], dx[kN], tab[(size_t)NTAB * kN];
   for (int d = 0; d < 3; d++) {
     const int N = D->GD[d];
+    D->hdx[d].resize(D->keep_geometry ? N : 0);
     for (int i = 0; i < N; i++)
       cw[i] = Para->CellWidth[d] ? Para->CellWidth[d][i] : (d < Para->GridRank ? Para->dx[d] : 1.0);
     for (int i = 0; i < N; i++)
       dx[i] = D->comoving && d < Para->GridRank ? D->a_sweep * cw[i] : cw[i];
+    // widths that the device has already (a handle's next call on its grid)
+    if (D->keep_geometry && !D->comoving) {
+      if (D->geometry[d] && memcmp(D->hdx[d].data(), dx, sizeof(double) * N) == 0) continue;
+      memcpy(D->hdx[d].data(), dx, sizeof(double) * N);
+    }
+    D->geometry[d] = false;
     build_tables(dx, N, tab);
     D->uni[d] = uniform_axis(dx, N, tab, D->kt[d]) ? 1 : 0;
     HIPCHK(hipMemcpyAsync(D->tab[d], tab, sizeof(double) * NTAB * (size_t)N,
@@ -699,6 +637,7 @@ int upload_geometry(hipPPMData *D, const hipPPMParameter *Para) {
       HIPCHK(hipMemcpyAsync(D->cwdt[d], cw, sizeof(double) * N, hipMemcpyHostToDevice,
                             D->stream));
     HIPCHK(hipStreamSynchronize(D->stream));  // the staging is reused for the next axis
+    D->geometry[d] = D->keep_geometry && !D->comoving;
   }
   return ENZO_PPM_SUCCESS;
 }
@@ -846,6 +785,7 @@ int hipPPMInitData(hipPPMData **Data, const hipPPMParameter *Para, void *stream)
     D = new (std::nothrow) hipPPMData();
     if (!D) return ENZO_PPM_ERR_ARGUMENT;
     *Data = D;
+    D->keep_geometry = true;
     HIPCHK(hipGetDevice(&D->device));
     for (int d = 0; d < 3; d++) D->GD[d] = (int)Para->GridDimension[d];
     D->cells = cells;
@@ -944,12 +884,6 @@ int hipPPMSetSubgridFluxes(hipPPMData *D, const hipPPMParameter *P, enzo_fluxes 
     D->hfaces[dim].clear();
     D->hface_sub[dim].clear();
     D->hface_side[dim].clear();
-    if (D->face_head[dim]) (void)hipFree(D->face_head[dim]);
-    if (D->faces[dim]) (void)hipFree(D->faces[dim]);
-    if (D->face_out[dim]) (void)hipFree(D->face_out[dim]);
-    D->face_head[dim] = nullptr;
-    D->faces[dim] = nullptr;
-    D->face_out[dim] = nullptr;
     D->face_total[dim] = 0;
     std::vector<int> head;
     long long total = 0;
@@ -960,15 +894,19 @@ int hipPPMSetSubgridFluxes(hipPPMData *D, const hipPPMParameter *P, enzo_fluxes 
     const std::vector<FaceRec> &sorted = D->hfaces[dim];
     D->face_total[dim] = total;
     if (total > 0) {
-      if (alloc_dev((void **)&D->face_head[dim], sizeof(int) * head.size()) ||
-          alloc_dev((void **)&D->faces[dim], sizeof(FaceRec) * sorted.size()) ||
-          alloc_dev((void **)&D->face_out[dim], sizeof(double) * total))
+      if (grow_dev(&D->face_head[dim], D->head_cap[dim], head.size()) ||
+          grow_dev(&D->faces[dim], D->rec_cap[dim], sorted.size()) ||
+          grow_dev(&D->face_out[dim], D->out_cap[dim], (size_t)total)) {
+        D->face_total[dim] = 0;
         return ENZO_PPM_ERR_HIP;
-      HIPCHK(hipMemcpy(D->face_head[dim], head.data(), sizeof(int) * head.size(),
-                       hipMemcpyHostToDevice));
-      HIPCHK(hipMemcpy(D->faces[dim], sorted.data(), sizeof(FaceRec) * sorted.size(),
-                       hipMemcpyHostToDevice));
+      }
+      // on the stream: sweeps queued before may still write the buffers kept
+      HIPCHK(hipMemcpyAsync(D->face_head[dim], head.data(), sizeof(int) * head.size(),
+                            hipMemcpyHostToDevice, D->stream));
+      HIPCHK(hipMemcpyAsync(D->faces[dim], sorted.data(), sizeof(FaceRec) * sorted.size(),
+                            hipMemcpyHostToDevice, D->stream));
       HIPCHK(hipMemsetAsync(D->face_out[dim], 0, sizeof(double) * total, D->stream));
+      HIPCHK(hipStreamSynchronize(D->stream));  // head leaves scope
     }
   }
   return ENZO_PPM_SUCCESS;
@@ -996,7 +934,7 @@ int hipPPMSaveSubgridFluxes(enzo_fluxes *SubgridFluxes[], enzo_int NumberOfSubgr
                              P->GridEndIndex[2] - P->GridStartIndex[2] + 1};
   std::vector<long long> f;
   slot_fields(P, f);
-  scatter_face_fluxes(h, D->hfaces[dir], D->hface_sub[dir], D->hface_side[dir], f, nact, (int)dir,
+  scatter_face_fluxes(h.data(), D->hfaces[dir], D->hface_sub[dir], D->hface_side[dir], f, nact, (int)dir,
                       SubgridFluxes);
   return ENZO_PPM_SUCCESS;
 }
@@ -1087,9 +1025,11 @@ int hipPPMSolvePPM_DE(const enzo_ppm_grid *g, const enzo_ppm_globals *gl, enzo_i
     const int dir = n % rank;
     if (nact[dir] <= 1) continue;
     st = launch_sweep(D, &Para, g->dtFixed, nullptr, dir);
-    if (st == ENZO_PPM_SUCCESS && NumberOfSubgrids > 0)
-      st = hipPPMSaveSubgridFluxes(SubgridFluxes, NumberOfSubgrids, ggs, D, &Para, dir);
   }
+  // (each axis has its own staging: read back once everything is queued)
+  for (int n = ixyz; n < ixyz + rank && st == ENZO_PPM_SUCCESS && NumberOfSubgrids > 0; n++)
+    if (nact[n % rank] > 1)
+      st = hipPPMSaveSubgridFluxes(SubgridFluxes, NumberOfSubgrids, ggs, D, &Para, n % rank);
   if (st == ENZO_PPM_SUCCESS) st = hipPPMGetBaryon(D, &Para, g->BaryonField);
   if (!Data) hipPPMDestroy(local);
   return st;

@@ -737,7 +737,7 @@ inline int build_face_records(const int GD[3], const hipPPMParameter *P,
 
 // Host: a grid's captured fluxes of one axis (staging `h`) into its
 // SubgridFluxes, with the velocity guards of Grid_[xyz]EulerSweep.C:343-357.
-inline void scatter_face_fluxes(const std::vector<double> &h, const std::vector<FaceRec> &recs,
+inline void scatter_face_fluxes(const double *h, const std::vector<FaceRec> &recs,
                                 const std::vector<int> &sub, const std::vector<int> &side,
                                 const std::vector<long long> &slot_field, const long long nact[3],
                                 int dim, enzo_fluxes *const *SubgridFluxes) {
@@ -749,7 +749,7 @@ inline void scatter_face_fluxes(const std::vector<double> &h, const std::vector<
       if (s >= S_VX && s <= S_VZ && (s - S_VX) != dim && nact[s - S_VX] <= 1) continue;
       enzo_float *out = side[r] == 0 ? F->LeftFluxes[slot_field[s]][dim] : F->RightFluxes[slot_field[s]][dim];
       if (!out) continue;
-      memcpy(out, h.data() + R.base + (size_t)s * R.nface, sizeof(double) * R.nface);
+      memcpy(out, h + R.base + (size_t)s * R.nface, sizeof(double) * R.nface);
     }
   }
 }

@@ -1,8 +1,11 @@
 // Host side of the host-array transfers (hipPPMSetBaryon / hipPPMGetBaryon
-// with the caller's pageable arrays): a small pool of host threads that
-// copies between the caller's memory and pinned staging buffers, so that
-// the host copy of one chunk overlaps the DMA of the previous one.
+// and their level forms, with the caller's pageable arrays): a small pool of
+// host threads that copies between the caller's memory and pinned staging
+// buffers, so that the host copy of one chunk overlaps the DMA of the
+// previous one.
 #pragma once
+
+#include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <atomic>
@@ -14,10 +17,16 @@
 
 namespace ppm {
 
-// memcpy split over the calling thread and up to 7 workers (pageable host
-// memory is copied at a few GB/s per thread; the DMA engine moves pinned
-// memory at ~57 GB/s).  One copy at a time per pool; copy() returns when
-// every byte is in place.
+// memcpy of several pieces split over the calling thread and up to 7 workers
+// (pageable host memory is copied at a few GB/s per thread; the DMA engine
+// moves pinned memory at ~57 GB/s).  One copy at a time per pool; copy()
+// returns when every byte is in place.
+struct CopyPiece {
+  char *dst;
+  const char *src;
+  size_t n;
+};
+
 class CopyPool {
  public:
   static CopyPool &get() {
@@ -25,19 +34,20 @@ class CopyPool {
     return pool;
   }
 
-  void copy(void *dst, const void *src, size_t n) {
+  void copy(const std::vector<CopyPiece> &pieces) {
+    size_t n = 0;
+    for (const CopyPiece &p : pieces) n += p.n;
     if (n < kMinParallel || workers_.empty()) {
-      std::memcpy(dst, src, n);
+      for (const CopyPiece &p : pieces) std::memcpy(p.dst, p.src, p.n);
       return;
     }
     std::lock_guard<std::mutex> one(busy_);  // callers from several threads take turns
     Job j;
-    j.dst = static_cast<char *>(dst);
-    j.src = static_cast<const char *>(src);
-    j.n = n;
     const size_t parts = 4 * (workers_.size() + 1);
-    j.slice = std::max<size_t>(kMinSlice, (n + parts - 1) / parts);
-    j.nslices = (n + j.slice - 1) / j.slice;
+    const size_t slice = std::max<size_t>(kMinSlice, (n + parts - 1) / parts);
+    for (const CopyPiece &p : pieces)
+      for (size_t off = 0; off < p.n; off += slice)
+        j.slices.push_back({p.dst + off, p.src + off, std::min(slice, p.n - off)});
     {
       std::lock_guard<std::mutex> lk(m_);
       job_ = &j;
@@ -51,13 +61,11 @@ class CopyPool {
   }
 
  private:
-  static constexpr size_t kMinParallel = size_t(1) << 20;
-  static constexpr size_t kMinSlice = size_t(256) << 10;
+  static constexpr size_t kMinParallel = size_t(512) << 10;
+  static constexpr size_t kMinSlice = size_t(128) << 10;
 
   struct Job {
-    char *dst = nullptr;
-    const char *src = nullptr;
-    size_t n = 0, slice = 0, nslices = 0;
+    std::vector<CopyPiece> slices;
     std::atomic<size_t> next{0};
     int users = 0;  // workers inside run(); guarded by m_
   };
@@ -79,9 +87,8 @@ class CopyPool {
   static void run(Job &j) {
     for (;;) {
       const size_t k = j.next.fetch_add(1);
-      if (k >= j.nslices) return;
-      const size_t off = k * j.slice, len = std::min(j.slice, j.n - off);
-      std::memcpy(j.dst + off, j.src + off, len);
+      if (k >= j.slices.size()) return;
+      std::memcpy(j.slices[k].dst, j.slices[k].src, j.slices[k].n);
     }
   }
 
@@ -113,6 +120,155 @@ class CopyPool {
   Job *job_ = nullptr;
   unsigned gen_ = 0;
   bool stop_ = false;
+};
+
+struct HostXfer {
+  char *dst;
+  const char *src;
+  size_t bytes;
+};
+
+// A ring of pinned buffers.  hipMemcpy from pageable arrays moves ~28 GB/s to
+// the device and ~18 GB/s back (the runtime stages them itself) and a small
+// one takes 10 us; here the pieces of a transfer go in chunks through the
+// ring, the host copy of each chunk overlapping the DMA of the others, which
+// runs at ~57 GB/s, and pieces that are neighbours on the device share one
+// DMA.  A transfer is cut into about four chunks, so that a single grid's
+// overlap too.
+class StageRing {
+ public:
+  static constexpr int kBufs = 3;
+  static constexpr size_t kMaxBytes = size_t(32) << 20;  // per pinned buffer
+  static constexpr size_t kMinChunk = size_t(1) << 20;
+
+  static size_t total(const std::vector<HostXfer> &xs) {
+    size_t t = 0;
+    for (const HostXfer &x : xs) t += x.bytes;
+    return t;
+  }
+  static size_t chunk_of(size_t bytes) {
+    return std::max(kMinChunk, std::min(kMaxBytes, (bytes / 4 + 4095) & ~size_t(4095)));
+  }
+
+  // buffers for transfers of up to `bytes`; false where they cannot be pinned
+  bool reserve(size_t bytes) {
+    const size_t want = chunk_of(bytes);
+    if (size_ >= want) return true;
+    release();
+    for (int b = 0; b < kBufs; b++)
+      if (hipHostMalloc(&buf_[b], want, hipHostMallocDefault) != hipSuccess ||
+          hipEventCreateWithFlags(&ev_[b], hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        release();
+        return false;
+      }
+    size_ = want;
+    return true;
+  }
+
+  // waits for the copies in flight and gives the buffers back
+  void release() {
+    for (int b = 0; b < kBufs; b++) {
+      if (busy_[b]) (void)hipEventSynchronize(ev_[b]);
+      busy_[b] = false;
+      if (ev_[b]) (void)hipEventDestroy(ev_[b]);
+      if (buf_[b]) (void)hipHostFree(buf_[b]);
+      ev_[b] = nullptr;
+      buf_[b] = nullptr;
+    }
+    size_ = 0;
+  }
+
+  // host -> device on `stream`; the caller's arrays may be reused on return
+  // (the DMA reads only the ring).  reserve() first.
+  hipError_t upload(hipStream_t stream, const std::vector<HostXfer> &xs) {
+    const size_t chunk = std::min(size_, chunk_of(total(xs)));
+    std::vector<CopyPiece> in;      // host copies into the current buffer
+    std::vector<HostXfer> out;      // and its DMAs (neighbours merged)
+    size_t pos = 0;
+    hipError_t e = hipSuccess;
+    auto close = [&]() {
+      if (!pos || e != hipSuccess) return;
+      CopyPool::get().copy(in);
+      for (const HostXfer &d : out)
+        if (e == hipSuccess) e = hipMemcpyAsync(d.dst, d.src, d.bytes, hipMemcpyHostToDevice, stream);
+      busy_[next_] = true;
+      if (e == hipSuccess) e = hipEventRecord(ev_[next_], stream);
+      next_ = (next_ + 1) % kBufs;
+      in.clear();
+      out.clear();
+      pos = 0;
+    };
+    for (const HostXfer &x : xs)
+      for (size_t off = 0; off < x.bytes && e == hipSuccess;) {
+        if (pos == chunk) close();
+        if (pos == 0 && (e == hipSuccess)) e = wait(next_);
+        if (e != hipSuccess) break;
+        const size_t n = std::min(chunk - pos, x.bytes - off);
+        in.push_back({at(pos), x.src + off, n});
+        if (!out.empty() && out.back().dst + out.back().bytes == x.dst + off) out.back().bytes += n;
+        else out.push_back({x.dst + off, at(pos), n});
+        pos += n;
+        off += n;
+      }
+    close();
+    return e;
+  }
+
+  // device -> host after the work queued on `stream`; complete on return
+  hipError_t download(hipStream_t stream, const std::vector<HostXfer> &xs) {
+    const size_t chunk = std::min(size_, chunk_of(total(xs)));
+    std::vector<CopyPiece> pend[kBufs];  // host copies out of each buffer
+    hipError_t e = hipSuccess;
+    auto drain = [&](int b) {
+      if (e == hipSuccess) e = wait(b);
+      if (e == hipSuccess) CopyPool::get().copy(pend[b]);
+      pend[b].clear();
+    };
+    size_t pos = 0, len0 = 0;
+    const char *src0 = nullptr;
+    auto dma = [&]() {
+      if (len0 && e == hipSuccess)
+        e = hipMemcpyAsync(at(pos - len0), src0, len0, hipMemcpyDeviceToHost, stream);
+      len0 = 0;
+    };
+    auto close = [&]() {
+      dma();
+      if (pos && e == hipSuccess) e = hipEventRecord(ev_[next_], stream);
+      busy_[next_] = busy_[next_] || pos;
+      if (pos) next_ = (next_ + 1) % kBufs;
+      pos = 0;
+    };
+    for (const HostXfer &x : xs)
+      for (size_t off = 0; off < x.bytes && e == hipSuccess;) {
+        if (pos == chunk) close();
+        if (pos == 0) drain(next_);
+        const size_t n = std::min(chunk - pos, x.bytes - off);
+        if (len0 && src0 + len0 != x.src + off) dma();
+        if (!len0) src0 = x.src + off;
+        pend[next_].push_back({x.dst + off, at(pos), n});
+        pos += n;
+        len0 += n;
+        off += n;
+      }
+    close();
+    for (int k = 0; k < kBufs; k++) drain((next_ + k) % kBufs);
+    return e;
+  }
+
+ private:
+  char *at(size_t pos) { return static_cast<char *>(buf_[next_]) + pos; }
+  hipError_t wait(int b) {
+    if (!busy_[b]) return hipSuccess;
+    busy_[b] = false;
+    return hipEventSynchronize(ev_[b]);
+  }
+
+  void *buf_[kBufs] = {nullptr, nullptr, nullptr};
+  hipEvent_t ev_[kBufs] = {nullptr, nullptr, nullptr};
+  bool busy_[kBufs] = {false, false, false};  // a copy into or out of it is queued, ev_ marks its end
+  int next_ = 0;
+  size_t size_ = 0;
 };
 
 }  // namespace ppm
