@@ -286,10 +286,11 @@ __device__ inline double pressure_dt_cell(const PresParams &Q, long long g) {
   double p = pressure_of(Q, g, Q.min_support);
   as_global(Q.pres)[g] = p;
   if (!Q.want_dt) return 1.0e20;
-  int i = (int)(g % Q.GD[0]);
-  long long r = g / Q.GD[0];
-  int j = (int)(r % Q.GD[1]);
-  int k = (int)(r / Q.GD[1]);
+  // (every index is below 1031^3 < 2^31: 32-bit divisions)
+  const unsigned r = (unsigned)g / (unsigned)Q.GD[0];
+  const int i = (int)((unsigned)g % (unsigned)Q.GD[0]);
+  const int j = (int)(r % (unsigned)Q.GD[1]);
+  const int k = (int)(r / (unsigned)Q.GD[1]);
   if (i < Q.st[0] || i > Q.en[0] || j < Q.st[1] || j > Q.en[1] || k < Q.st[2] || k > Q.en[2])
     return 1.0e20;
   // calc_dt's pressure uses minimum-support coefficient 0
@@ -627,9 +628,9 @@ __device__ inline void prep_item(const FlatParams &F, long long gid) {
     return;
   }
   if (!F.iflatten) return;
-  const long long k = gid - F.N;
-  const int ncell = F.i2 - F.i1 + 3;
-  if (k >= (long long)ncell * F.n_outer) return;
+  const unsigned ncell = (unsigned)(F.i2 - F.i1 + 3);
+  if (gid - F.N >= (long long)ncell * F.n_outer) return;
+  const unsigned k = (unsigned)(gid - F.N);  // below 1031^2 + 2 * 1031
   const int outer = (int)(k / ncell);
   const int cell = F.i1 - 1 + (int)(k % ncell);
   as_global(F.flat)[(long long)outer * F.N + (cell - 1)] = flat_value(F, outer, cell);

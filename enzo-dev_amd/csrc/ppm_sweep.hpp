@@ -2163,24 +2163,23 @@ struct FlatParams {
 PPM_HD double flat_value(const FlatParams &F, int outer, int cell) {
   const int rax = (F.dim + 1) % 3, oax = (F.dim + 2) % 3;
   const bool de = F.iflatten >= 2;  // types 2 and 3 read density and energy too
+  // line 1 of the slice: cell cc at base + (cc - 1) * st.  Type 1 reads p
+  // within 3 cells and u within 2, the others both (and d, e) within 4.
+  const int st3[3] = {1, F.GD[0], F.GD[0] * F.GD[1]};
+  const int base = outer * st3[oax], st = st3[F.dim];
+  (void)rax;
   double pv[9], uv[9], dv[9], ev[9];
   for (int k = -4; k <= 4; k++) {
     int cc = cell + k;
-    if (cc < 1 || cc > F.N) {
-      pv[k + 4] = 1.0; uv[k + 4] = 0.0; dv[k + 4] = 1.0; ev[k + 4] = 0.0;
-      continue;
-    }
-    int c[3];
-    c[F.dim] = cc - 1;
-    c[rax] = 0;
-    c[oax] = outer;
-    long long g = ((long long)c[2] * F.GD[1] + c[1]) * F.GD[0] + c[0];
+    pv[k + 4] = 1.0; uv[k + 4] = 0.0; dv[k + 4] = 1.0; ev[k + 4] = 0.0;
+    if (cc < 1 || cc > F.N || (!de && (k < -3 || k > 3))) continue;
+    const long long g = base + (cc - 1) * st;
     PPM_ASSERT(g >= 0 && g < F.cells);
     const auto A = as_global(F.A);
     pv[k + 4] = as_global(F.pres)[g];
-    uv[k + 4] = A[(S_VX + F.dim) * F.cells + g];
-    dv[k + 4] = de ? A[S_D * F.cells + g] : 1.0;
-    ev[k + 4] = de ? A[S_E * F.cells + g] : 0.0;
+    if (de || (k >= -2 && k <= 2)) uv[k + 4] = A[(S_VX + F.dim) * F.cells + g];
+    if (de) dv[k + 4] = A[S_D * F.cells + g];
+    if (de) ev[k + 4] = A[S_E * F.cells + g];
   }
   auto P = [&](int x) { PPM_ASSERT(x - cell >= -4 && x - cell <= 4); return pv[x - cell + 4]; };
   auto U = [&](int x) { PPM_ASSERT(x - cell >= -4 && x - cell <= 4); return uv[x - cell + 4]; };
