@@ -39,8 +39,8 @@ SIMDS, VALU_CYCLES_PER_INST, CLOCK_HZ = 1024, 4, 2.4e9
 # rocprofv3 counts of one 256^3 sweep of the turbulent workload with the
 # current build (profiles/ppm_sweep_kernel_turbulent256.md): wave-level VALU
 # instructions, waves, and the FP64 add / mul / fma / transcendental parts
-VALU_PER_SWEEP_256, WAVES_PER_SWEEP_256 = 1.232e9, 345840
-F64_ADD, F64_MUL, F64_FMA, F64_TRANS = 0.168e9, 0.210e9, 0.218e9, 0.0355e9
+VALU_PER_SWEEP_256, WAVES_PER_SWEEP_256 = 0.966e9, 345840
+F64_ADD, F64_MUL, F64_FMA, F64_TRANS = 0.164e9, 0.197e9, 0.160e9, 0.0223e9
 
 
 def parse():
@@ -131,9 +131,9 @@ def cpu_baseline(n, threads, repeats=5):
 
 
 def level_solver_rates(lib, ngrids, steps, cfl=0.4):
-    """The same AMR level batched with RiemannSolver HLL and HLLC (whole
-    pencils in one-pencil workgroups sized to the level's pencils): steps
-    of the level's Courant dt after two untimed ones."""
+    """The same AMR level batched with RiemannSolver HLL and HLLC (their
+    fluxes in the sweep tiles): steps of the level's Courant dt after two
+    untimed ones."""
     import numpy as np
     from enzo_ppm import problems
     from enzo_ppm.level import Level
@@ -616,8 +616,8 @@ def main():
                                      "2.4 GHz; frac = the share of the kernel's time the "
                                      "SIMDs spend issuing VALU instructions"}
     if a.solver_steps > 0:
-        # RiemannSolver HLL / HLLC on the same workload: whole pencils in the
-        # one-pencil workgroups (not the metric; the two-shock solver is)
+        # RiemannSolver HLL / HLLC on the same workload (not the metric; the
+        # two-shock solver is)
         print("bench: HLL and HLLC solvers", file=sys.stderr, flush=True)
         out["other_solvers"] = {}
         for name, rs in (("hll", 1), ("hllc", 4)):
